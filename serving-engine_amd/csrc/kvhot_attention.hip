@@ -34,7 +34,9 @@
 //    mask from q_pos_offset; tiles past the work-group's last query are never
 //    loaded.
 //  * attn_generic_kernel<T>: VALU kernel for fp32 (exact fp32 arithmetic) and
-//    for shapes the MFMA kernels do not cover.
+//    for shapes the MFMA kernels do not cover (query groups of more than 16
+//    heads, other head_dims, blocks that are not whole 16-token slices,
+//    unaligned rows).
 #include "kvhot_internal.h"
 
 #include <algorithm>
@@ -71,7 +73,7 @@ struct AttnArgs {
   int64_t num_partials;
   int64_t num_blocks;
   int32_t Hq, Hkv, G, bs;
-  int32_t part_tokens, max_parts;
+  int32_t part_tokens, max_parts, wave_slices;  // no schedule
   float scale_log2;
   int32_t causal;
   int32_t D;        // head_dim (generic kernel)
@@ -157,32 +159,19 @@ __device__ inline __amdgpu_buffer_rsrc_t block_rsrc(const void* base, int bytes)
 #endif
 constexpr int kKvLoadPolicy = KVHOT_KV_LOAD_POLICY;
 
-// Loads N dwords (N in {2, 4, 8}) at byte offset off (+ uniform soff) of r.
+// Loads N dwords (N in {2, 3, 4, 8}) at byte offset off (+ uniform soff) of r.
 template <int N>
 __device__ inline void buffer_dwords(__amdgpu_buffer_rsrc_t r, int off, int soff, uint32_t* out) {
   if constexpr (N == 2) {
     const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, kKvLoadPolicy));
     out[0] = v.x; out[1] = v.y;
+  } else if constexpr (N == 3) {
+    const u32x3 v = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(r, off, soff, kKvLoadPolicy));
+    out[0] = v.x; out[1] = v.y; out[2] = v.z;
   } else {
 #pragma unroll
     for (int c = 0; c < N / 4; ++c) {
       const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16 * c, soff, kKvLoadPolicy));
-      out[4 * c + 0] = v.x; out[4 * c + 1] = v.y;
-      out[4 * c + 2] = v.z; out[4 * c + 3] = v.w;
-    }
-  }
-}
-
-// Loads N dwords (N in {2, 4, 8}) from a 16-bit element pointer.
-template <int N>
-__device__ inline void load_dwords(const uint16_t* p, uint32_t* out) {
-  if constexpr (N == 2) {
-    u32x2 v = *reinterpret_cast<const u32x2*>(p);
-    out[0] = v.x; out[1] = v.y;
-  } else {
-#pragma unroll
-    for (int c = 0; c < N / 4; ++c) {
-      u32x4 v = *reinterpret_cast<const u32x4*>(p + 8 * c);
       out[4 * c + 0] = v.x; out[4 * c + 1] = v.y;
       out[4 * c + 2] = v.z; out[4 * c + 3] = v.w;
     }
@@ -215,8 +204,16 @@ constexpr float kLazyRescale = 15.f;
 
 
 // One wavefront's attention state and key loop.
-template <class TT, int D, int NM>
+// SP: probabilities enter the PV product as two 16-bit values, the rounded
+// one and what the rounding left (P = hi + lo to 2^-17 in bf16, 2^-22 in
+// fp16), so that an output carries its own rounding only: against fp64, bf16
+// outputs of random inputs are off by 0.0017 in relative L2, as with fp32
+// probabilities, and by 0.0023 with rounded ones.  It costs a second PV
+// product (1.5 times the MFMAs) and 5 VALU instructions per pair of
+// probabilities.
+template <class TT, int D, int NM, bool SP = false>
 struct WaveAttn {
+  static constexpr int NP = SP ? 2 * NM : NM;  // packed P operands: hi of every m-row tile, then lo
   static constexpr int NC = D / 32;
   static constexpr int EPL = D / 16;  // head_dim values per lane per V row; PV MFMAs per tile
   static constexpr int VW = EPL / 2;
@@ -225,7 +222,7 @@ struct WaveAttn {
   int n, g;
   // m-row s*16 + n of this lane: causal limit (key positions up to it are visible) and validity
   int kvh_;                  // the work's kv head (uniform)
-  int qbase_, lg_g_;         // causal limit of query 0 (INT_MAX: none), log2 G (uniform)
+  int qbase_, inv_g_;        // causal limit of query 0 (INT_MAX: none), ceil(2^16 / G) (uniform)
   int qpos[NM];
   bool mval[NM];
   u32x4 qf[NM][NC];  // Q as the B operand of S^T = K . Q^T
@@ -242,7 +239,7 @@ struct WaveAttn {
     kvh_ = kvh;
     const int G = a.G;
     qbase_ = a.causal ? off + q0 : INT_MAX;
-    lg_g_ = __builtin_ctz(static_cast<unsigned>(G));
+    inv_g_ = (65536 + G - 1) / G;
 #pragma unroll
     for (int s = 0; s < NM; ++s) {
       const int i = 16 * s + n;
@@ -267,9 +264,10 @@ struct WaveAttn {
 
   // Query (within the block), query head and causal limit of m-row s of
   // this lane, recomputed where needed rather than held in registers through
-  // the loop (G a power of two).
+  // the loop.  (i * ceil(2^16 / G)) >> 16 is i / G exactly: i < 64 and
+  // G <= 16, so the product is off by less than 64 / 2^16 < 1 / G.)
   __device__ int qlimit(int s) const {
-    return mval[s] ? (qbase_ == INT_MAX ? INT_MAX : qbase_ + ((16 * s + n) >> lg_g_)) : -1;
+    return mval[s] ? (qbase_ == INT_MAX ? INT_MAX : qbase_ + (((16 * s + n) * inv_g_) >> 16)) : -1;
   }
   __device__ int row_query(const AttnArgs& a, int s) const { return (16 * s + n) / a.G; }
   __device__ int row_head(const AttnArgs& a, int s) const { return kvh_ * a.G + (16 * s + n) % a.G; }
@@ -351,7 +349,7 @@ struct WaveAttn {
       }
     }
     // Online softmax (base 2); P^T packed as the B operand of O^T += V^T . P^T.
-    u32x2 pb[NM];
+    u32x2 pb[NP];
 #pragma unroll
     for (int s = 0; s < NM; ++s) {
       float mx = fmaxf(fmaxf(sc[s][0], sc[s][1]), fmaxf(sc[s][2], sc[s][3]));
@@ -366,6 +364,7 @@ struct WaveAttn {
       l[s] = l[s] * corr + ((pr[0] + pr[1]) + (pr[2] + pr[3]));
       m[s] = mnew;
       pb[s] = u32x2{TT::pack2(pr[0], pr[1]), TT::pack2(pr[2], pr[3])};
+      if constexpr (SP) pb[NM + s] = u32x2{rest2(pr[0], pr[1], pb[s].x), rest2(pr[2], pr[3], pb[s].y)};
 #pragma unroll
       for (int e = 0; e < EPL; ++e) o[s][e] *= corr;
     }
@@ -377,8 +376,16 @@ struct WaveAttn {
       const u32x2 vt = {__builtin_amdgcn_perm(T.v[1][w], T.v[0][w], sel),
                         __builtin_amdgcn_perm(T.v[3][w], T.v[2][w], sel)};
 #pragma unroll
-      for (int s = 0; s < NM; ++s) o[s][e] = TT::mfma16(vt, pb[s], o[s][e]);
+      for (int s = 0; s < NM; ++s) {
+        o[s][e] = TT::mfma16(vt, pb[s], o[s][e]);
+        if constexpr (SP) o[s][e] = TT::mfma16(vt, pb[NM + s], o[s][e]);
+      }
     }
+  }
+
+  // What rounding x and y to the packed pair hi left, packed.
+  __device__ static uint32_t rest2(float x, float y, uint32_t hi) {
+    return TT::pack2(x - TT::low_float(hi), y - TT::high_float(hi));
   }
 
   // ---- 32-key LDS tiles (PreTile layout, rows of Tile::RB bytes) ----
@@ -434,7 +441,7 @@ struct WaveAttn {
 
   // P = 2^(S sl - m) as the packed B operand of the PV product, and this
   // lane's sums of P per m-row (ls, not yet added to l).
-  __device__ void probs(float sl, const f32x4 (&sc)[NM][2], u32x4 (&pb)[NM], float (&ls)[NM]) const {
+  __device__ void probs(float sl, const f32x4 (&sc)[NM][2], u32x4 (&pb)[NP], float (&ls)[NM]) const {
 #pragma unroll
     for (int s = 0; s < NM; ++s) {
       float p[2][4];
@@ -445,6 +452,9 @@ struct WaveAttn {
       ls[s] = ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) + ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3]));
       pb[s] = u32x4{TT::pack2(p[0][0], p[0][1]), TT::pack2(p[0][2], p[0][3]),
                     TT::pack2(p[1][0], p[1][1]), TT::pack2(p[1][2], p[1][3])};
+      if constexpr (SP)
+        pb[NM + s] = u32x4{rest2(p[0][0], p[0][1], pb[s].x), rest2(p[0][2], p[0][3], pb[s].y),
+                           rest2(p[1][0], p[1][1], pb[s].z), rest2(p[1][2], p[1][3], pb[s].w)};
     }
   }
 
@@ -464,22 +474,6 @@ struct WaveAttn {
 #pragma unroll
       for (int e = 0; e < EPL; ++e) o[s][e] *= corr;
     }
-  }
-
-  // Softmax of a tile with no masked key: P formed with the current
-  // references first, so that everything up to the rare move of a
-  // reference is one branch-free block the scheduler can interleave with
-  // MFMAs, and formed again after a move.
-  __device__ void softmax_nomask(float sl, const f32x4 (&sc)[NM][2], u32x4 (&pb)[NM]) {
-    float mloc[NM], ls[NM];
-    const bool need = lazy_check(sc, mloc);
-    probs(sl, sc, pb, ls);
-    if (__builtin_amdgcn_ballot_w64(need) != 0) {
-      move_refs(sl, mloc);
-      probs(sl, sc, pb, ls);
-    }
-#pragma unroll
-    for (int s = 0; s < NM; ++s) l[s] += ls[s];
   }
 
   // V^T operands of a tile, read with ds_read_b64_tr_b16.  Within a 16-lane
@@ -510,7 +504,7 @@ struct WaveAttn {
   // 16e + i (lane (n, g) holds 16e + 4g + j of m-row n).  va holds blocks
   // 0 .. VB-1 on entry.
   template <class Tile>
-  __device__ void pv_lds(const char* vt, u32x4 (&va)[VB], const u32x4 (&pb)[NM]) {
+  __device__ void pv_lds(const char* vt, u32x4 (&va)[VB], const u32x4 (&pb)[NP]) {
     // (va is overwritten when EPL > VB.)
 #pragma unroll
     for (int e0 = 0; e0 < EPL; e0 += VB) {
@@ -518,7 +512,7 @@ struct WaveAttn {
 #pragma unroll
       for (int e = 0; e < VB; ++e)
 #pragma unroll
-        for (int s = 0; s < NM; ++s) o[s][e0 + e] = TT::mfma(va[e], pb[s], o[s][e0 + e]);
+        for (int s = 0; s < NP; ++s) o[s % NM][e0 + e] = TT::mfma(va[e], pb[s], o[s % NM][e0 + e]);
     }
   }
 
@@ -564,7 +558,7 @@ struct WaveAttn {
           sc[s][h][j] = (tk < kstop && tk <= qlimit(s)) ? sc[s][h][j] : -INFINITY;
         }
   }
-  __device__ void softmax_tile(float sl, f32x4 (&sc)[NM][2], bool mask, int ts, int kstop, u32x4 (&pb)[NM]) {
+  __device__ void softmax_tile(float sl, f32x4 (&sc)[NM][2], bool mask, int ts, int kstop, u32x4 (&pb)[NP]) {
     if (mask) mask_tile(sc, ts, kstop);
     float mloc[NM], ls[NM];
     if (__builtin_amdgcn_ballot_w64(lazy_check(sc, mloc)) != 0) move_refs(sl, mloc);
@@ -620,12 +614,11 @@ struct WaveAttn {
 #endif
 
 // Waves per kv head in grid mode for a partition of nslices slices: the
-// smallest power of two up to W that keeps each wave near
-// KVHOT_SLICES_PER_WAVE slices and leaves no more than Hkv kv heads to a
-// work-group (no idle waves).
-__host__ __device__ inline int decode_splits(int nslices, int W, int Hkv) {
+// smallest power of two up to W that keeps each wave near wave_slices slices
+// and leaves no more than Hkv kv heads to a work-group (no idle waves).
+__host__ __device__ inline int decode_splits(int nslices, int W, int Hkv, int wave_slices) {
   int S = 1;
-  while (S < W && (S * KVHOT_SLICES_PER_WAVE < nslices || W / S > Hkv)) S *= 2;
+  while (S < W && (S * wave_slices < nslices || W / S > Hkv)) S *= 2;
   return S;
 }
 
@@ -654,7 +647,8 @@ __device__ inline int wave_max_int(int x) {
 // MR: the launch list gives a work-group more ranges than waves (fixed
 // partitions, decode_ranges); otherwise one range per wave, and P is W.
 // VB: KVHOT_VERIFY_BLOCKS (below).
-template <class TT, int D, int W, bool MR, bool VB>
+// SP: WaveAttn's.
+template <class TT, int D, int W, bool MR, bool VB, bool SP>
 __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& a, const int4* sched, int bx, int by,
                                                                 int bz) {
   extern __shared__ float smem[];
@@ -705,7 +699,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
     if (p >= np) return;
     const int kbeg = p * PT;
     const int nsl = max((min(ke_r, kbeg + PT) - kbeg + 15) / 16, 0);
-    const int Sp = decode_splits(nsl, W, a.Hkv);
+    const int Sp = decode_splits(nsl, W, a.Hkv, a.wave_slices);
     const int HW = W / Sp;
     if (static_cast<int>(bx) * HW >= a.Hkv) return;
     const int h = bx * HW + wave / Sp;
@@ -761,7 +755,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   // query position passed to the m-row setup is kend - 1.
   int krow = valid ? row : -1, kkvh = kvh, kpart = part, kkend = kend;
 
-  WaveAttn<TT, D, 1> wa;
+  WaveAttn<TT, D, 1, SP> wa;
   wa.setup(a, lane, valid ? kvh : 0, qs, 0, valid ? 1 : 0, kend - 1);
   KVSlice<D> T;
   int i = s0;              // slice whose loads are in flight, if `have`
@@ -860,6 +854,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   };
   int slot = wave;
   bool used = false;       // the slot holds work
+  constexpr int FV = (D / 16) % 4 == 0 ? 2 : 1;  // float pairs per store of flush (D = 96: rows of 6 values)
   auto flush = [&]() {
     float lt[1];
     wa.row_sums(lt);
@@ -869,10 +864,14 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
 #pragma unroll
       for (int j = 0; j < 4; ++j)
 #pragma unroll
-        for (int e = 0; e < D / 16; e += 4)
-          *reinterpret_cast<f32x4*>(dst + (D / 16) * (4 * wa.g + j) + e) =
-              f32x4{wa.o[0][e][j] * inv, wa.o[0][e + 1][j] * inv, wa.o[0][e + 2][j] * inv,
-                    wa.o[0][e + 3][j] * inv};
+        for (int e = 0; e < D / 16; e += 2 * FV)
+          if constexpr (FV == 2)
+            *reinterpret_cast<f32x4*>(dst + (D / 16) * (4 * wa.g + j) + e) =
+                f32x4{wa.o[0][e][j] * inv, wa.o[0][e + 1][j] * inv, wa.o[0][e + 2][j] * inv,
+                      wa.o[0][e + 3][j] * inv};
+          else
+            *reinterpret_cast<f32x2*>(dst + (D / 16) * (4 * wa.g + j) + e) =
+                f32x2{wa.o[0][e][j] * inv, wa.o[0][e + 1][j] * inv};
       if (wa.g == 0) sl[slot * G + wa.n] = lt[0] > 0.f ? wa.m[0] + __log2f(lt[0]) : -INFINITY;
     }
     if (lane == 0) {
@@ -1174,10 +1173,10 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   }
 }
 
-template <class TT, int D, int W, bool MR = false, bool VB = false>
+template <class TT, int D, int W, bool MR = false, bool VB = false, bool SP = false>
 __global__ void __launch_bounds__(64 * W)
 attn_decode_kernel(const AttnArgs a) {
-  decode_wg<TT, D, W, MR, VB>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
+  decode_wg<TT, D, W, MR, VB, SP>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Combines the parts of split decode segments: (row, kv head) pieces that
@@ -1394,12 +1393,28 @@ struct PreTile {
   static constexpr int RB = 2 * D;               // bytes per key row
   static constexpr int BYTES = kPreKeys * RB;    // bytes per K (or V) tile
   static constexpr int CHUNKS = kPreKeys * CPR;  // chunks per tile
-  // DMA instructions per issuing wave (K or V): kPreIssuers waves issue a tile.
-  static constexpr int NI = CHUNKS / (64 * kPreIssuers);
-  static_assert(CHUNKS % (64 * kPreIssuers) == 0, "a tile splits evenly over the issuing waves");
+  // The kPreIssuers issuing waves share a tile's DMA: each copies a quarter
+  // of K and a quarter of V, or where a tile is not four equal runs of 64
+  // chunks (D = 96: 6) each copies one 16-key half of K or of V.
+  static constexpr bool ONE_POOL = CHUNKS % (64 * kPreIssuers) != 0;
+  // DMA instructions per issuing wave and pool.
+  static constexpr int NI = ONE_POOL ? CHUNKS / 128 : CHUNKS / (64 * kPreIssuers);
+  static_assert(CHUNKS % 128 == 0, "a 16-key half is whole DMA instructions");
   // 128-byte rows (D = 64) share a 256-byte bank line in pairs.
   __host__ __device__ static constexpr int swz(int r) { return D == 64 ? (r >> 1) & 7 : r & 15; }
-  __host__ __device__ static constexpr int offset(int r, int lc) { return r * RB + 16 * (lc ^ swz(r)); }
+  // D = 96: 192-byte rows start at 4 bank offsets, 12 (r & 3) chunks mod 16,
+  // and a row's 12 chunks are rotated by 0 to 3 places by r / 4: 16 rows at
+  // one logical chunk (K), and the two-chunk pieces of rows 4g .. 4g+3 of two
+  // lane groups (V^T), fall in distinct banks.
+  __host__ __device__ static constexpr int rot(int r) { return ((r >> 1) & 2) | ((r >> 3) & 1); }
+  // Physical chunk of logical chunk lc of row r, and the inverse.
+  __host__ __device__ static constexpr int phys(int r, int lc) {
+    return D == 96 ? (lc + rot(r) >= CPR ? lc + rot(r) - CPR : lc + rot(r)) : lc ^ swz(r);
+  }
+  __host__ __device__ static constexpr int logical(int r, int pc) {
+    return D == 96 ? (pc - rot(r) < 0 ? pc - rot(r) + CPR : pc - rot(r)) : pc ^ swz(r);
+  }
+  __host__ __device__ static constexpr int offset(int r, int lc) { return r * RB + 16 * phys(r, lc); }
 };
 
 // s_waitcnt vmcnt(N) alone (expcnt and lgkmcnt at their no-wait maximum).
@@ -1430,12 +1445,12 @@ __device__ inline void half_barrier() {
 
 // One prefill work-group: launch-list unit bx (prefill units at sched), or
 // without a launch list grid work-group (bx, by, bz).
-template <class TT, int D, int NM>
+template <class TT, int D, int NM, bool SP>
 __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs& a, const int4* sched, int bx, int by,
                                                                  int bz) {
   (void)by;
   using Tile = PreTile<D>;
-  using WA = WaveAttn<TT, D, NM>;
+  using WA = WaveAttn<TT, D, NM, SP>;
   constexpr int PW = prefill_waves(D);
   // Ring slots, K tile then V tile.  Separate arrays: the compiler can tell
   // that reads of one slot do not alias the DMA into another, and so does
@@ -1487,7 +1502,7 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   } else {
     row = bz;
     kvh = bx % a.Hkv;
-    qblk = bx / a.Hkv;
+    qblk = (static_cast<int>(gridDim.x) - 1 - bx) / a.Hkv;  // the longest key ranges start first
   }
   row = __builtin_amdgcn_readfirstlane(row);
   kvh = __builtin_amdgcn_readfirstlane(kvh);
@@ -1524,18 +1539,21 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   const int qpos_min = causal ? off + q0 : INT_MAX;
 
   // DMA: issuing wave w (the leading group), instruction i fills chunks
-  // 64 (NI w + i) .. of a tile; all of a wave's chunks lie in the one 16-key
-  // half hw.  Lane L's chunk is physical chunk pc of row pr; it loads logical
-  // chunk pc ^ swz(pr) of that key.
+  // 64 (NI cw + i) .. of a tile, cw = w (or w % 2 with ONE_POOL: waves 0 and
+  // 1 copy K, 2 and 3 V); all of a wave's chunks lie in the one 16-key half
+  // hw.  Lane L's chunk is physical chunk pc of row pr; it loads that key's
+  // logical chunk.
   constexpr int NI = Tile::NI;
+  constexpr bool ONE_POOL = Tile::ONE_POOL;
   const bool issuer = wave < kPreIssuers;
-  const int hw = __builtin_amdgcn_readfirstlane(issuer ? (64 * NI * wave) / (16 * Tile::CPR) : 0);
+  const int cw = ONE_POOL ? wave & 1 : wave;
+  const int hw = __builtin_amdgcn_readfirstlane(issuer ? (64 * NI * cw) / (16 * Tile::CPR) : 0);
   uint32_t koff[NI], voff[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int p = 64 * (NI * (issuer ? wave : 0) + i) + lane;
+    const int p = 64 * (NI * (issuer ? cw : 0) + i) + lane;
     const int pr = p / Tile::CPR, pc = p % Tile::CPR;
-    const int lc = pc ^ Tile::swz(pr);
+    const int lc = Tile::logical(pr, pc);
     koff[i] = 2u * ((pr & 15) * static_cast<uint32_t>(a.k_st) + 8u * lc);
     voff[i] = 2u * ((pr & 15) * static_cast<uint32_t>(a.v_st) + 8u * lc);
   }
@@ -1580,12 +1598,24 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
         ++nblk;
       }
     }
-    char* dst = slot(S) + 1024 * NI * wave;
-    const rsrc_words_t kr = rsrc_words(kb, nrk), vr = rsrc_words(vb, nrv);
+    char* dst = slot(S) + 1024 * NI * cw;
+    if constexpr (ONE_POOL) {
+      if (wave < 2) {
+        const rsrc_words_t kr = rsrc_words(kb, nrk);
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      dma16_asm(kr, dst + 1024 * i, koff[i]);
-      dma16_asm(vr, dst + Tile::BYTES + 1024 * i, voff[i]);
+        for (int i = 0; i < NI; ++i) dma16_asm(kr, dst + 1024 * i, koff[i]);
+      } else {
+        const rsrc_words_t vr = rsrc_words(vb, nrv);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) dma16_asm(vr, dst + Tile::BYTES + 1024 * i, voff[i]);
+      }
+    } else {
+      const rsrc_words_t kr = rsrc_words(kb, nrk), vr = rsrc_words(vb, nrv);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        dma16_asm(kr, dst + 1024 * i, koff[i]);
+        dma16_asm(vr, dst + Tile::BYTES + 1024 * i, voff[i]);
+      }
     }
   };
 
@@ -1596,8 +1626,11 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   // per tile, pinning the two waves of a SIMD half a tile apart, measured
   // 187.5 us against 182.6 for one, on the mixed workload's prefill rows
   // with 8-wave work-groups.)
-  constexpr int PER_TILE = 2 * NI;  // DMA instructions per issuing wave and tile
-  constexpr int LEAD = WA::NC <= 4 ? 3 : 2;
+  constexpr int PER_TILE = ONE_POOL ? NI : 2 * NI;  // DMA instructions per issuing wave and tile
+  // (SP: the second P operand takes the registers of the pipelined phase's
+  // second set of scores.)
+  constexpr bool kVAhead = WA::NC <= 4 && !SP;
+  constexpr int LEAD = kVAhead ? 3 : 2;
   const int ntiles = (kend_g - k0 + kPreKeys - 1) / kPreKeys;
   // Tiles [0, nfull) have no key masked for this wave; tiles from kend on
   // have no key it sees.
@@ -1630,7 +1663,6 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   }
   half_barrier();
 
-  constexpr bool kVAhead = WA::NC <= 4;
   if constexpr (kVAhead) {
     // head_dim 64 and 128, software-pipelined: phase t reads K(t+1) and
     // V^T(t), runs QK(t+1) while it forms P(t) from the scores QK(t) left in
@@ -1664,7 +1696,7 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
       const char* vt = slot(S) + Tile::BYTES;
       const char* kn = slot((S + 1) & 3);
       u32x4 va[WA::VB];
-      u32x4 pb[NM];
+      u32x4 pb[WA::NP];
       f32x4 scn[NM][2];
       // References first (rare move, before the block), then one block:
       // K(t+1) and V^T(t) reads, QK(t+1) and P(t).
@@ -1714,7 +1746,7 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
       if (t >= nfull) wa.mask_tile(scc, ts, kend);
       const char* vt = slot(S) + Tile::BYTES;
       u32x4 va[WA::VB];
-      u32x4 pb[NM];
+      u32x4 pb[WA::NP];
       wa.template read_vt<Tile>(vt, 0, va);
       wa.softmax_tile(sl, scc, false, ts, kend, pb);
       wa.template pv_lds<Tile>(vt, va, pb);
@@ -1737,12 +1769,12 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
       default: last(std::integral_constant<int, 3>{}, nlast); break;
     }
   } else {
-    // head_dim 256 (K operands in halves, V^T read in the phase of its PV):
+    // head_dim 256, and SP (K operands in halves, V^T read in the phase of its PV):
     // phase t issues tile t+2 into the slot of tile t-2, reads K(t) half by
     // half around PV(t-1), runs QK(t) and forms P(t); before the barrier an
     // issuing wave waits for its part of tile t+1 (vmcnt <= PER_TILE while
     // tile t+2 is in flight).
-    u32x4 pb[NM];      // P of the previous tile, for its PV
+    u32x4 pb[WA::NP];  // P of the previous tile, for its PV
     u32x4 va[WA::VB];  // its V^T operands
     bool pv_due = false;
     auto step = [&](auto S_, int t) {
@@ -1752,12 +1784,15 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
       const bool live = t < ntiles && ts < kend;
       f32x4 sc[NM][2];
       u32x4 kh[WA::NC];
-      if (live) wa.template k_operands<Tile>(slot(S), 0, kh);
+      // (SP at head_dim 256 has no registers for K beside V^T.)
+      constexpr bool kEarly = !(SP && D == 256);
+      if (kEarly && live) wa.template k_operands<Tile>(slot(S), 0, kh);
       if (pv_due) {
         wa.template read_vt<Tile>(slot((S + 3) & 3) + Tile::BYTES, 0, va);
         wa.template pv_lds<Tile>(slot((S + 3) & 3) + Tile::BYTES, va, pb);
       }
       if (live) {
+        if (!kEarly) wa.template k_operands<Tile>(slot(S), 0, kh);
         wa.qk_ops(kh, 0, sc);
         wa.template k_operands<Tile>(slot(S), 1, kh);
         wa.qk_ops(kh, 1, sc);
@@ -1797,10 +1832,10 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
 }
 
 // Two waves per SIMD at every head_dim (at most 256 VGPRs a wave).
-template <class TT, int D, int NM>
+template <class TT, int D, int NM, bool SP = false>
 __global__ void __launch_bounds__(64 * prefill_waves(D)) __attribute__((amdgpu_waves_per_eu(2)))
 attn_prefill_kernel(const AttnArgs a) {
-  prefill_wg<TT, D, NM>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
+  prefill_wg<TT, D, NM, SP>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // ----------------------------------------------------------- VALU kernel --
@@ -1961,25 +1996,53 @@ static int64_t partial_bytes(int64_t G, int64_t D) { return G * (D + 1) * 4; }
 
 struct Plan {
   bool mfma = false;     // the MFMA kernels take this shape
+  bool lists = false;    // ... and launch lists are built for it
   bool grid_ok = false;  // ... also without a schedule (partition count fits the grid)
   int waves = 0;         // waves per decode work-group
   int part_tokens = 0;   // keys per decode partition (no schedule)
+  int wave_slices = KVHOT_SLICES_PER_WAVE;  // slices a decode wave is given (no schedule)
   int max_parts = 1;
   int64_t partials = 0;  // split-K partials without a schedule
   int64_t workspace_bytes(int64_t G, int64_t D) const { return partials * partial_bytes(G, D); }
 };
 
+// 16-row tiles of (query, head) pairs per prefill wave: O^T takes 64 VGPRs
+// and Q 32 (D = 96: 48 and 24), so two waves fit on a SIMD.
+#ifndef KVHOT_PRE_NM128
+#define KVHOT_PRE_NM128 2
+#endif
+constexpr int prefill_nm(int64_t D) { return D == 64 ? 4 : (D == 128 || D == 96 ? KVHOT_PRE_NM128 : 1); }
+
+// Shapes of the MFMA kernels: query groups of 1 to 16 heads (a decode wave's
+// 16 m-rows; a prefill wave takes 16 NM / G whole queries, so a group that is
+// not a power of two leaves at most 2 of 32 m-rows empty for G <= 7).
 static bool mfma_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dtype) {
   if (dtype != KVHOT_BF16 && dtype != KVHOT_F16) return false;
-  if (D != 64 && D != 128 && D != 256) return false;
-  if (bs % 16 != 0) return false;
-  const int64_t G = Hq / Hkv;
-  return G == 1 || G == 2 || G == 4 || G == 8 || G == 16;
+  if (D != 64 && D != 96 && D != 128 && D != 256) return false;
+  return bs % 16 == 0 && Hq / Hkv <= 16;
 }
 
+// Shapes launch lists are built for; the others run from the grid, with
+// probabilities split in two (WaveAttn's SP), and without split-K when the
+// caller brings no workspace for it.  24 query heads on 8 kv heads, 13 decode
+// rows of up to 1500 keys and 5 chunks of up to 300: 925 us with one VALU wave
+// per (query, head), 49.5 us here.
+static bool list_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dtype) {
+  const int64_t G = Hq / Hkv;
+  return mfma_shape_ok(Hq, Hkv, D, bs, dtype) && D != 96 && (G & (G - 1)) == 0;
+}
+
+// Queries of one (row, kv head) a prefill work-group takes.
+static int64_t prefill_queries(int64_t D, int64_t G) { return prefill_waves(D) * (16 * prefill_nm(D) / G); }
+
+// Waves a grid launch without launch lists tries to fill: 8 on each CU.
+constexpr int64_t kGridWaves = 256 * 8;
+
 // Without a schedule, decode rows are cut into partitions of part_tokens keys
-// (0: W * KVHOT_SLICES_PER_WAVE slices, so no wave walks more than that many)
-// and the grid enumerates (head group, partition, row).
+// (0: W * wave_slices slices, so no wave walks more than that many) and the
+// grid enumerates (head group, partition, row).  wave_slices is
+// KVHOT_SLICES_PER_WAVE; for shapes that never have launch lists, fewer (at
+// least 2) when the rows' slices would not fill kGridWaves waves.
 static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
                       int64_t Hkv, int64_t D, int64_t bs, int64_t part_tokens,
                       int dtype) {
@@ -1987,8 +2050,13 @@ static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
   pl.mfma = mfma_shape_ok(Hq, Hkv, D, bs, dtype);
   if (!pl.mfma || max_q < 1) return pl;
   pl.waves = decode_waves(Hq / Hkv, D);
-  pl.part_tokens = part_tokens > 0 ? static_cast<int>(part_tokens)
-                                   : 16 * pl.waves * KVHOT_SLICES_PER_WAVE;
+  pl.lists = list_shape_ok(Hq, Hkv, D, bs, dtype);
+  if (!pl.lists) {
+    const int64_t slices = rows * Hkv * ((max_k + 15) / 16);
+    pl.wave_slices = static_cast<int>(
+        std::max<int64_t>(2, std::min<int64_t>(KVHOT_SLICES_PER_WAVE, slices / kGridWaves)));
+  }
+  pl.part_tokens = part_tokens > 0 ? static_cast<int>(part_tokens) : 16 * pl.waves * pl.wave_slices;
   const int64_t parts = std::max<int64_t>((max_k + pl.part_tokens - 1) / pl.part_tokens, 1);
   if (parts > 65535) return pl;
   pl.grid_ok = true;
@@ -1996,13 +2064,6 @@ static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
   if (pl.max_parts > 1) pl.partials = rows * Hkv * pl.max_parts;
   return pl;
 }
-
-// 16-row tiles of (query, head) pairs per prefill wave: O^T takes 64 VGPRs
-// and Q 32 at every head_dim, so two waves fit on a SIMD.
-#ifndef KVHOT_PRE_NM128
-#define KVHOT_PRE_NM128 2
-#endif
-constexpr int prefill_nm(int64_t D) { return D == 64 ? 4 : (D == 128 ? KVHOT_PRE_NM128 : 1); }
 
 // Decode work-groups the current device holds at once, times their waves
 // (one work-group on each of 256 CUs when no device can be queried).
@@ -2444,7 +2505,7 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
   for (int64_t r = 0; r < rows; ++r) {
     const int64_t qlen = q_lens[r], klen = k_lens[r], off = q_offs[r];
     if (qlen < 2) continue;
-    const int64_t qpw = prefill_waves(D) * 16 * prefill_nm(D) / G;  // queries per work-group
+    const int64_t qpw = prefill_queries(D, G);
     for (int64_t qb = 0; qb * qpw < qlen; ++qb) {
       const int64_t q0 = qb * qpw, nq = std::min(qpw, qlen - q0);
       const int64_t kend = std::max<int64_t>(causal ? std::min(klen, off + q0 + nq) : klen, 0);
@@ -2464,7 +2525,7 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
   pre.swap(wide);
 }
 
-template <class TT, int D, int W>
+template <class TT, int D, int W, bool SP>
 static void launch_decode(const AttnArgs& a, int64_t rows, int64_t n_dec, hipStream_t stream) {
   AttnArgs da = a;
   da.dec_ranges = a.sched && a.dec_ranges > W && n_dec % a.dec_ranges == 0 ? a.dec_ranges : W;
@@ -2481,17 +2542,23 @@ static void launch_decode(const AttnArgs& a, int64_t rows, int64_t n_dec, hipStr
   };
   // One instantiation per mode, so that the common one carries none of the
   // others' code.
-  const bool mr = da.dec_ranges > W, vb = a.verify && a.sched;
-  if (mr && vb) go(attn_decode_kernel<TT, D, W, true, true>);
-  else if (mr) go(attn_decode_kernel<TT, D, W, true, false>);
-  else if (vb) go(attn_decode_kernel<TT, D, W, false, true>);
-  else go(attn_decode_kernel<TT, D, W, false, false>);
+  if constexpr (SP) {
+    go(attn_decode_kernel<TT, D, W, false, false, true>);
+  } else {
+    const bool mr = da.dec_ranges > W, vb = a.verify && a.sched;
+    if (mr && vb) go(attn_decode_kernel<TT, D, W, true, true>);
+    else if (mr) go(attn_decode_kernel<TT, D, W, true, false>);
+    else if (vb) go(attn_decode_kernel<TT, D, W, false, true>);
+    else go(attn_decode_kernel<TT, D, W, false, false>);
+  }
 }
 
-template <class TT, int D>
+// SP: a shape without launch lists (a.sched null).
+template <class TT, int D, bool SP>
 static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_q, int64_t n_dec,
                         int64_t n_pre, int64_t n_merge, int64_t n_pfx, hipStream_t stream) {
   constexpr int NM = prefill_nm(D);
+  if constexpr (!SP)
   if (a.sched && n_pfx > 0) {
     // Shared-prefix units, the first n_pfx of the prefill section, before
     // anything else on the caller's stream: the decode launch folds in the
@@ -2510,27 +2577,27 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
   const bool dec = !a.sched || n_dec > 0;
   const bool pre = a.sched ? n_pre > n_pfx : max_q >= 2;
   if (pre) {
-    const int64_t qpw = prefill_waves(D) * 16 * NM / a.G;
+    const int64_t qpw = prefill_queries(D, a.G);
     const int64_t nqb = (max_q + qpw - 1) / qpw;
     dim3 grid = a.sched ? dim3(static_cast<uint32_t>(n_pre - n_pfx))
                         : dim3(static_cast<uint32_t>(a.Hkv * nqb), 1u, static_cast<uint32_t>(rows));
     AttnArgs pa = a;
     if (a.sched) pa.sched = a.sched + 2 * (n_dec + n_pfx);
-    hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM>), grid, dim3(64 * prefill_waves(D)), 0, stream, pa);
+    hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM, SP>), grid, dim3(64 * prefill_waves(D)), 0, stream, pa);
   }
   if (dec) {
     bool launched = false;
 #if KVHOT_MAX_DECODE_WAVES >= 16
     if constexpr (D <= 128) {
       if (waves == 16) {
-        launch_decode<TT, D, 16>(a, rows, n_dec, stream);
+        launch_decode<TT, D, 16, SP>(a, rows, n_dec, stream);
         launched = true;
       }
     }
 #else
     (void)waves;
 #endif
-    if (!launched) launch_decode<TT, D, 8>(a, rows, n_dec, stream);
+    if (!launched) launch_decode<TT, D, 8, SP>(a, rows, n_dec, stream);
   }
   if (a.sched ? n_merge > 0 : (!a.sched || n_dec > 0) && a.max_parts > 1) {
     dim3 mgrid = a.sched ? dim3(static_cast<uint32_t>(n_merge))
@@ -2591,10 +2658,10 @@ extern "C" int64_t kvhot_paged_attention_schedule(
   int64_t partials = 0;
   const Plan pl = make_plan(num_rows, max_q, max_k, num_q_heads, num_kv_heads, head_dim,
                             block_size, partition_tokens, dtype);
-  if (pl.mfma) {
+  if (pl.lists) {
     const int64_t G = num_q_heads / num_kv_heads;
     const int64_t groups = resident_decode_waves(dtype, head_dim, pl.waves, G) / pl.waves;
-    const int64_t prefix_queries = prefill_waves(head_dim) * 16 * prefill_nm(head_dim) / G;  // per prefill work-group
+    const int64_t prefix_queries = prefill_queries(head_dim, G);  // per prefill work-group
     const int ranges = decode_ranges(pl.waves, G, head_dim, partition_tokens > 0);
     if (plan_decode(q_lens, k_lens, q_pos_offsets, q_starts, block_table, bt_row_stride, block_size,
                     num_rows, num_kv_heads, is_causal, pl.waves, ranges, groups, partition_tokens,
@@ -2699,10 +2766,10 @@ static int paged_attention_impl(
   a.verify = (attn_flags & KVHOT_VERIFY_BLOCKS) ? 1 : 0;
   a.D = static_cast<int32_t>(head_dim);
   a.total_q = total_query;
-  const int64_t n_dec = schedule ? num_decode_units : 0;
-  const int64_t n_pre = schedule ? num_prefill_units : 0;
-  const int64_t n_mrg = schedule ? num_merge_units : 0;
-  const int64_t n_pfx = schedule ? num_prefix_units : 0;
+  int64_t n_dec = schedule ? num_decode_units : 0;
+  int64_t n_pre = schedule ? num_prefill_units : 0;
+  int64_t n_mrg = schedule ? num_merge_units : 0;
+  int64_t n_pfx = schedule ? num_prefix_units : 0;
   if (schedule && (n_dec < 0 || n_pre < 0 || n_mrg < 0 || n_dec > 0x7fffffff ||
                    n_pre > 0x7fffffff || n_mrg > 0x7fffffff || schedule_workspace_bytes < 0 ||
                    n_pfx < 0 || n_pfx > n_pre))
@@ -2714,6 +2781,11 @@ static int paged_attention_impl(
 
   Plan pl = make_plan(num_rows, max_q_len, max_k_len, num_q_heads, num_kv_heads, head_dim,
                       block_size, partition_tokens, dtype);
+  if (!pl.lists) {  // a launch list means nothing for this shape
+    schedule = nullptr;
+    a.sched = a.merge_units = nullptr;
+    n_dec = n_pre = n_mrg = n_pfx = 0;
+  }
   if (!schedule && !pl.grid_ok) pl.mfma = false;
   if (schedule && pl.mfma && n_dec % pl.waves != 0)
     return set_error(KVHOT_EINVAL, "paged_attention: decode schedule is not whole work-groups");
@@ -2734,6 +2806,12 @@ static int paged_attention_impl(
   }
   if (pl.mfma) {
     const int64_t pb = partial_bytes(a.G, head_dim);
+    if (!pl.lists && pl.partials > 0 && (!workspace || workspace_bytes < pl.workspace_bytes(a.G, head_dim))) {
+      // Without room for partials every row is one partition.
+      pl.part_tokens = static_cast<int>(std::max<int64_t>((max_k_len + 15) / 16 * 16, 16));
+      pl.max_parts = 1;
+      pl.partials = 0;
+    }
     if (schedule && (n_mrg > 0 || n_pfx > 0) && schedule_workspace_bytes < pb)
       return set_error(KVHOT_EINVAL, "paged_attention: a schedule with merge or prefix units needs partials");
     const int64_t need = schedule ? (n_mrg > 0 || n_pfx > 0 ? schedule_workspace_bytes : 0)
@@ -2749,23 +2827,31 @@ static int paged_attention_impl(
     if (!schedule) {
       a.part_tokens = pl.part_tokens;
       a.max_parts = pl.max_parts;
+      a.wave_slices = pl.wave_slices;
     }
     // A launch list of fixed partitions groups its decode ranges as the
     // planner did (the same partition_tokens is passed to both calls; with
     // another value the ranges come in groups of one per wave, which gives
     // the same results).
     a.dec_ranges = schedule ? decode_ranges(pl.waves, a.G, head_dim, partition_tokens > 0) : pl.waves;
-#define KVHOT_MFMA(TT, DD) \
-  launch_mfma<TT, DD>(a, pl.waves, num_rows, max_q_len, n_dec, n_pre, n_mrg, n_pfx, s)
-    if (dtype == KVHOT_BF16) {
-      if (head_dim == 64) KVHOT_MFMA(BF16, 64);
-      else if (head_dim == 128) KVHOT_MFMA(BF16, 128);
-      else KVHOT_MFMA(BF16, 256);
-    } else {
-      if (head_dim == 64) KVHOT_MFMA(F16, 64);
-      else if (head_dim == 128) KVHOT_MFMA(F16, 128);
-      else KVHOT_MFMA(F16, 256);
-    }
+#define KVHOT_MFMA(TT, DD, SP) \
+  launch_mfma<TT, DD, SP>(a, pl.waves, num_rows, max_q_len, n_dec, n_pre, n_mrg, n_pfx, s)
+#define KVHOT_MFMA_D(TT)                                                              \
+  do {                                                                                \
+    if (pl.lists) {                                                                   \
+      if (head_dim == 64) KVHOT_MFMA(TT, 64, false);                                  \
+      else if (head_dim == 128) KVHOT_MFMA(TT, 128, false);                           \
+      else KVHOT_MFMA(TT, 256, false);                                                \
+    } else {                                                                          \
+      if (head_dim == 64) KVHOT_MFMA(TT, 64, true);                                   \
+      else if (head_dim == 96) KVHOT_MFMA(TT, 96, true);                              \
+      else if (head_dim == 128) KVHOT_MFMA(TT, 128, true);                            \
+      else KVHOT_MFMA(TT, 256, true);                                                 \
+    }                                                                                 \
+  } while (0)
+    if (dtype == KVHOT_BF16) KVHOT_MFMA_D(BF16);
+    else KVHOT_MFMA_D(F16);
+#undef KVHOT_MFMA_D
 #undef KVHOT_MFMA
     return launch_status("paged_attention");
   }
@@ -2868,6 +2954,9 @@ extern "C" int kvhot_paged_attention_noalloc(
     need = kvhot_paged_attention_workspace_bytes(num_rows, total_query, max_q_len, max_k_len, num_q_heads,
                                                  num_kv_heads, head_dim, block_size, partition_tokens, dtype);
     if (need < 0) return set_error(static_cast<int>(need), "paged_attention_noalloc: bad sizes");
+    // (Shapes without launch lists run unsplit where their partials do not fit.)
+    if (need > KVHOT_NOALLOC_SCRATCH_BYTES && !list_shape_ok(num_q_heads, num_kv_heads, head_dim, block_size, dtype))
+      need = 0;
   }
   if (need > KVHOT_NOALLOC_SCRATCH_BYTES)
     return set_error(KVHOT_EWORKSPACE, "paged_attention_noalloc: the call needs " + std::to_string(need) +

@@ -40,6 +40,7 @@ inline int64_t dtype_size(int dtype) {
 constexpr int kWave = 64;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -64,6 +65,9 @@ struct BF16 {
   __device__ static inline uint32_t pack2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
   }
+  // The values of a packed pair.
+  __device__ static inline float low_float(uint32_t p) { return __uint_as_float(p << 16); }
+  __device__ static inline float high_float(uint32_t p) { return __uint_as_float(p & 0xffff0000u); }
   __device__ static inline f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(
         __builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -84,6 +88,12 @@ struct F16 {
   }
   __device__ static inline uint32_t pack2(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, f16x2));
+  }
+  __device__ static inline float low_float(uint32_t p) {
+    return static_cast<float>(__builtin_bit_cast(f16x2, p).x);
+  }
+  __device__ static inline float high_float(uint32_t p) {
+    return static_cast<float>(__builtin_bit_cast(f16x2, p).y);
   }
   __device__ static inline f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(

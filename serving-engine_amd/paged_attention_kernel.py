@@ -186,7 +186,7 @@ def paged_flash_attention(q, k_cache, v_cache, metadata, num_q_heads, num_kv_hea
     stream = _lib.stream_handle(device)
     plan = _schedule(metadata, device, num_q_heads, num_kv_heads, head_dim, block_size, pt,
                      is_causal, dtype)
-    if plan is not None:
+    if plan is not None and plan[1] + plan[2] > 0:
         sched, n_dec, n_pre, n_mrg, need, n_pfx = plan
     else:
         sched, n_dec, n_pre, n_mrg, n_pfx = None, 0, 0, 0, 0
