@@ -33,10 +33,11 @@
 //    the QK of the next tile runs beside the softmax of this one.  Causal
 //    mask from q_pos_offset; tiles past the work-group's last query are never
 //    loaded.
-//  * attn_generic_kernel<T>: VALU kernel for fp32 (exact fp32 arithmetic) and
-//    for shapes the MFMA kernels do not cover (query groups of more than 16
-//    heads, other head_dims, blocks that are not whole 16-token slices,
-//    unaligned rows).
+//  * fp32: the decode kernel with WaveAttn<F32, ...> (v_mfma_f32_16x16x4_f32,
+//    operands straight from global memory) and attn_prefill_f32_kernel.
+//  * attn_generic_kernel<T>: VALU kernel for shapes the MFMA kernels do not
+//    cover (query groups of more than 16 heads, other head_dims, blocks that
+//    are not whole 16-token slices, unaligned rows).
 #include "kvhot_internal.h"
 
 #include <algorithm>
@@ -213,6 +214,7 @@ constexpr float kLazyRescale = 15.f;
 // probabilities.
 template <class TT, int D, int NM, bool SP = false>
 struct WaveAttn {
+  using Slice = KVSlice<D>;
   static constexpr int NP = SP ? 2 * NM : NM;  // packed P operands: hi of every m-row tile, then lo
   static constexpr int NC = D / 32;
   static constexpr int EPL = D / 16;  // head_dim values per lane per V row; PV MFMAs per tile
@@ -567,7 +569,224 @@ struct WaveAttn {
     for (int s = 0; s < NM; ++s) l[s] += ls[s];
   }
 
+  // Normalised O of m-row n, fp32, to row dst (head_dim order): the layout
+  // compute_slice leaves O in.
+  __device__ void store_slot(float* dst, float inv) const {
+    constexpr int FV = EPL % 4 == 0 ? 4 : 2;  // values per store (D = 96: 6 per row)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int e = 0; e < EPL; e += FV) {
+        float* p = dst + EPL * (4 * g + j) + e;
+        if constexpr (FV == 4)
+          *reinterpret_cast<f32x4*>(p) =
+              f32x4{o[0][e][j] * inv, o[0][e + 1][j] * inv, o[0][e + 2][j] * inv, o[0][e + 3][j] * inv};
+        else
+          *reinterpret_cast<f32x2*>(p) = f32x2{o[0][e][j] * inv, o[0][e + 1][j] * inv};
+      }
+  }
+
   // Row sums over the four lane groups that share an m-row.
+  __device__ void row_sums(float (&ltot)[NM]) const {
+#pragma unroll
+    for (int s = 0; s < NM; ++s) {
+      const float t = l[s] + __shfl_xor(l[s], 16, kWave);
+      ltot[s] = t + __shfl_xor(t, 32, kWave);
+    }
+  }
+};
+
+// ---------------------------------------------------------------- fp32 --
+// fp32 rows on v_mfma_f32_16x16x4_f32, which multiplies and adds in fp32.
+// One element of k per lane means any order of k does, as long as both
+// operands share it, so nothing is transposed and no LDS is used:
+//  * S^T = K . Q^T: lane (n, g) holds dims 16c + 4g .. +3 of K row n and of
+//    Q m-row n (16-byte loads); element i of chunk c is step (c, i).
+//  * O^T += V^T . P^T: step j covers keys 4g + j, g = 0..3: B is the score
+//    register j as it stands, A is element e of V row 4g + j, loaded by lane
+//    n at head_dim dim(e, n).
+// A slice is 2 * D / 4 MFMAs of 32 cycles per 16 m-rows: at head_dim 128 a
+// CU's four SIMDs consume K/V at 32 bytes per cycle, 19 TB/s over the chip,
+// so decode rows are bound by HBM; prefill rows are bound by the MFMAs.
+// At head_dim 256, K, V, Q and O together pass 256 registers: V is loaded
+// after QK, into K's.
+// Measured against one VALU wave per (query, head): 64 decode rows of 128 to
+// 2048 tokens (32 / 8 heads, D = 128) 1934 -> 172 us, two rows of 30,000
+// 26.7 ms -> 102 us (4.8 TB/s).
+template <int D>
+struct KVSlice32 {
+  static constexpr bool kLateV = D == 256;
+  f32x4 k[D / 16];            // token n, dims 16c + 4g .. +3
+  float v[kLateV ? 1 : 4][D / 16];  // token 4g+j, dims dim(e, n)
+  const float* vb;            // kLateV: V base of the block and slice offset (uniform)
+  int vs;
+  bool live;
+};
+
+template <int D, int NM>
+struct WaveAttn<F32, D, NM, false> {
+  using Slice = KVSlice32<D>;
+  static constexpr bool kLateV = Slice::kLateV;
+  static constexpr int NC = D / 16;
+  static constexpr int EPL = D / 16;
+  static constexpr int V4 = D / 64;  // 16-byte loads per V row per lane; D % 64 == 32 adds one of 8 bytes
+
+  int n, g;
+  int qpos[NM];
+  bool mval[NM];
+  f32x4 qf[NM][NC];
+  float m[NM], l[NM];
+  f32x4 o[NM][EPL];  // lane (n, g): head_dim dim(e, 4g + j) of m-row n
+
+  // Head_dim of element e of lane n's V loads.
+  __device__ static constexpr int dim(int e, int n) {
+    return e < 4 * V4 ? 64 * (e / 4) + 4 * n + e % 4 : 64 * V4 + 2 * n + (e - 4 * V4);
+  }
+
+  // As the 16-bit wave's.
+  __device__ void setup(const AttnArgs& a, int lane, int kvh, int64_t qs, int q0, int nq, int off) {
+    n = lane & 15;
+    g = lane >> 4;
+#pragma unroll
+    for (int s = 0; s < NM; ++s) {
+      const int i = 16 * s + n;
+      const int mq = i / a.G, mh = kvh * a.G + i % a.G;
+      mval[s] = mq < nq && qs + q0 + mq < a.total_q;
+      qpos[s] = mval[s] ? (a.causal ? off + q0 + mq : INT_MAX) : -1;
+      const float* qp = static_cast<const float*>(a.q) + (qs + q0 + mq) * a.q_st + static_cast<int64_t>(mh) * a.q_sh;
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        qf[s][c] = mval[s] ? *reinterpret_cast<const f32x4*>(qp + 16 * c + 4 * g) : f32x4{0.f, 0.f, 0.f, 0.f};
+      m[s] = -INFINITY;
+      l[s] = 0.f;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) o[s][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  }
+
+  __device__ void load_v(const AttnArgs& a, const float* vb, int vs, bool live, float (&v)[4][EPL]) const {
+    const __amdgpu_buffer_rsrc_t vr = block_rsrc(vb, live ? static_cast<int>(4 * a.v_sb) : 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int row = 4 * (4 * g + j) * static_cast<int>(a.v_st);
+#pragma unroll
+      for (int c = 0; c < V4; ++c) {
+        const f32x4 x = __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, row + 256 * c + 16 * n, vs, kKvLoadPolicy));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][4 * c + i] = x[i];
+      }
+      if constexpr (D % 64 != 0) {
+        const f32x2 x = __builtin_bit_cast(
+            f32x2, __builtin_amdgcn_raw_buffer_load_b64(vr, row + 256 * V4 + 8 * n, vs, kKvLoadPolicy));
+        v[j][4 * V4] = x.x;
+        v[j][4 * V4 + 1] = x.y;
+      }
+    }
+  }
+
+  // The slice at token bo of the block whose K and V rows of this kv head
+  // start at kb and vb (uniform); nothing is read unless live.
+  __device__ void load_slice_from(const AttnArgs& a, const float* kb, const float* vb, int bo, Slice& T,
+                                  bool live = true) const {
+    const __amdgpu_buffer_rsrc_t kr = block_rsrc(kb, live ? static_cast<int>(4 * a.k_sb) : 0);
+    const int ks = 4 * bo * static_cast<int>(a.k_st);
+    const int vs = 4 * bo * static_cast<int>(a.v_st);
+    const int k_lane = 4 * (n * static_cast<int>(a.k_st) + 4 * g);
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      T.k[c] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(kr, k_lane + 64 * c, ks, kKvLoadPolicy));
+    if constexpr (kLateV) {
+      T.vb = vb;
+      T.vs = vs;
+      T.live = live;
+    } else {
+      load_v(a, vb, vs, live, T.v);
+    }
+  }
+  __device__ void load_slice(const AttnArgs& a, int kvh, int64_t id, int bo, Slice& T, bool live = true) const {
+    load_slice_from(a, static_cast<const float*>(a.k) + static_cast<int64_t>(kvh) * a.k_sh + id * a.k_sb,
+                    static_cast<const float*>(a.v) + static_cast<int64_t>(kvh) * a.v_sh + id * a.v_sb, bo, T, live);
+  }
+
+  // Folds keys ts..ts+15 into the online softmax, masked as the 16-bit
+  // wave's compute_slice.
+  __device__ void compute_slice(const AttnArgs& a, int ts, int kstop, int qpos_min, Slice& T) {
+    f32x4 sc[NM];
+#pragma unroll
+    for (int s = 0; s < NM; ++s) {
+      // Two chains: MFMAs of one accumulator wait for each other.
+      f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+#pragma unroll
+        for (int i = 0; i < 4; i += 2) {
+          acc0 = F32::mfma4(T.k[c][i], qf[s][c][i], acc0);
+          acc1 = F32::mfma4(T.k[c][i + 1], qf[s][c][i + 1], acc1);
+        }
+      sc[s] = acc0 + acc1;
+    }
+    float late[kLateV ? 4 : 1][EPL];
+    if constexpr (kLateV) {
+      __builtin_amdgcn_sched_barrier(0);  // not before K's registers are free
+      load_v(a, T.vb, T.vs, T.live, late);
+    }
+    const bool tail = ts + 16 > kstop;
+    const bool full = !tail && ts + 15 <= qpos_min;
+#pragma unroll
+    for (int s = 0; s < NM; ++s) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float x = sc[s][j] * a.scale_log2;
+        if (!full) {
+          const int tk = ts + 4 * g + j;
+          x = (tk < kstop && tk <= qpos[s]) ? x : -INFINITY;
+        }
+        sc[s][j] = x;
+      }
+      float mx = fmaxf(fmaxf(sc[s][0], sc[s][1]), fmaxf(sc[s][2], sc[s][3]));
+      mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
+      mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+      const float mnew = fmaxf(m[s], mx);
+      const float muse = mnew == -INFINITY ? 0.f : mnew;
+      const float corr = F32::exp2(m[s] - muse);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) sc[s][j] = F32::exp2(sc[s][j] - muse);
+      l[s] = l[s] * corr + ((sc[s][0] + sc[s][1]) + (sc[s][2] + sc[s][3]));
+      m[s] = mnew;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) o[s][e] *= corr;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // Keys past the end may hold any bit pattern; zero them so 0 * V stays 0.
+      const bool ok = !tail || ts + 4 * g + j < kstop;
+#pragma unroll
+      for (int e = 0; e < EPL; ++e) {
+        float v;
+        if constexpr (kLateV) v = late[j][e];
+        else v = T.v[j][e];
+        v = ok ? v : 0.f;
+#pragma unroll
+        for (int s = 0; s < NM; ++s) o[s][e] = F32::mfma4(v, sc[s][j], o[s][e]);
+      }
+    }
+  }
+
+  // O of m-row tile s times f, to row dst (head_dim order).
+  __device__ void store_row(float* dst, int s, float f) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+      for (int e = 0; e < 4 * V4; e += 4)
+        *reinterpret_cast<f32x4*>(dst + dim(e, 4 * g + j)) =
+            f32x4{o[s][e][j] * f, o[s][e + 1][j] * f, o[s][e + 2][j] * f, o[s][e + 3][j] * f};
+      if constexpr (D % 64 != 0)
+        *reinterpret_cast<f32x2*>(dst + dim(4 * V4, 4 * g + j)) = f32x2{o[s][4 * V4][j] * f, o[s][4 * V4 + 1][j] * f};
+    }
+  }
+  __device__ void store_slot(float* dst, float inv) const { store_row(dst, 0, inv); }
+
   __device__ void row_sums(float (&ltot)[NM]) const {
 #pragma unroll
     for (int s = 0; s < NM; ++s) {
@@ -652,7 +871,7 @@ template <class TT, int D, int W, bool MR, bool VB, bool SP>
 __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& a, const int4* sched, int bx, int by,
                                                                 int bz) {
   extern __shared__ float smem[];
-  using st = uint16_t;
+  using st = typename TT::storage;
   // Wave-uniform values are pinned to SGPRs with readfirstlane: derived from
   // threadIdx they would otherwise count as divergent, putting block ids and
   // buffer descriptors in VGPRs (a waterfall loop around every load).
@@ -755,9 +974,11 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   // query position passed to the m-row setup is kend - 1.
   int krow = valid ? row : -1, kkvh = kvh, kpart = part, kkend = kend;
 
-  WaveAttn<TT, D, 1, SP> wa;
+  using WA = WaveAttn<TT, D, 1, SP>;
+  using Slice = typename WA::Slice;
+  WA wa;
   wa.setup(a, lane, valid ? kvh : 0, qs, 0, valid ? 1 : 0, kend - 1);
-  KVSlice<D> T;
+  Slice T;
   int i = s0;              // slice whose loads are in flight, if `have`
   bool have = nsl > 0;     // the first slice of the range is taken without a claim
 #if KVHOT_DECODE_DEPTH < 2
@@ -854,25 +1075,13 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   };
   int slot = wave;
   bool used = false;       // the slot holds work
-  constexpr int FV = (D / 16) % 4 == 0 ? 2 : 1;  // float pairs per store of flush (D = 96: rows of 6 values)
   auto flush = [&]() {
     float lt[1];
     wa.row_sums(lt);
     if (wa.mval[0]) {
       const float inv = lt[0] > 0.f ? 1.f / lt[0] : 0.f;
-      float* dst = so + (static_cast<int64_t>(slot) * G + wa.n) * D;
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int e = 0; e < D / 16; e += 2 * FV)
-          if constexpr (FV == 2)
-            *reinterpret_cast<f32x4*>(dst + (D / 16) * (4 * wa.g + j) + e) =
-                f32x4{wa.o[0][e][j] * inv, wa.o[0][e + 1][j] * inv, wa.o[0][e + 2][j] * inv,
-                      wa.o[0][e + 3][j] * inv};
-          else
-            *reinterpret_cast<f32x2*>(dst + (D / 16) * (4 * wa.g + j) + e) =
-                f32x2{wa.o[0][e][j] * inv, wa.o[0][e + 1][j] * inv};
-      if (wa.g == 0) sl[slot * G + wa.n] = lt[0] > 0.f ? wa.m[0] + __log2f(lt[0]) : -INFINITY;
+      wa.store_slot(so + (static_cast<int64_t>(slot) * G + wa.n) * D, inv);
+      if (wa.g == 0) sl[slot * G + wa.n] = lt[0] > 0.f ? wa.m[0] + TT::log2(lt[0]) : -INFINITY;
     }
     if (lane == 0) {
       skey[4 * slot + 0] = krow;
@@ -972,7 +1181,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   // slice and issues its block-table load, then refills the computed buffer
   // with iz.  iz's entry was loaded before the newer buffer's K/V, so waiting
   // for it leaves that buffer in flight (vector loads complete in order).
-  KVSlice<D> T1;
+  Slice T1;
   int ix = i, iy = 0, iz = 0, zraw = 0;
   bool hx = have, hy = false, hz = false;
   int cv = wave;           // range being claimed from
@@ -1003,7 +1212,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   // issued on every path (no bytes when nothing was claimed): the waits the
   // compiler places before a compute then always leave the other buffer's
   // loads in flight.
-  auto half = [&](KVSlice<D>& X, int& ix_, bool& hx_) {
+  auto half = [&](Slice& X, int& ix_, bool& hx_) {
     if (hx_) {
       wa.compute_slice(a, 16 * ix_, kkend, INT_MAX, X);
       used = true;
@@ -1087,7 +1296,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
       if (mx != -INFINITY) {
         for (uint64_t b = slots; b; b &= b - 1) {
           const int w = __builtin_ctzll(b);
-          const float wt = fast_exp2(sl[w * G + hh] - mx);
+          const float wt = TT::exp2(sl[w * G + hh] - mx);
           lsum += wt;
           acc += wt * *reinterpret_cast<const f32x4*>(so + (static_cast<int64_t>(w) * G + hh) * D + d0);
         }
@@ -1112,12 +1321,12 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
             cm = fmaxf(cm, lp[k]);
           }
           if (cm == -INFINITY) continue;
-          const float sc = mx == -INFINITY ? 0.f : fast_exp2(mx - cm);
+          const float sc = mx == -INFINITY ? 0.f : TT::exp2(mx - cm);
           acc *= sc;
           lsum *= sc;
 #pragma unroll
           for (int k = 0; k < kFoldBatch; ++k) {
-            const float wt = lp[k] == -INFINITY ? 0.f : fast_exp2(lp[k] - cm);
+            const float wt = lp[k] == -INFINITY ? 0.f : TT::exp2(lp[k] - cm);
             lsum += wt;
             acc += wt * ov[k];
           }
@@ -1126,11 +1335,10 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
       }
       const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
       const int h = mkvh * G + hh;
-      const float lse2 = lsum > 0.f ? mx + __log2f(lsum) : -INFINITY;
+      const float lse2 = lsum > 0.f ? mx + TT::log2(lsum) : -INFINITY;
       if (mnp == 1 || mfold) {
         st* dp = static_cast<st*>(a.o) + mqs * a.o_st + static_cast<int64_t>(h) * a.o_sh + d0;
-        *reinterpret_cast<u32x2*>(dp) =
-            u32x2{TT::pack2(acc.x * inv, acc.y * inv), TT::pack2(acc.z * inv, acc.w * inv)};
+        TT::store4(dp, acc * inv);
         if (a.lse && d0 == 0) a.lse[mqs * a.l_st + static_cast<int64_t>(h) * a.l_sh] = lse2 * kLn2;
       } else {
         *reinterpret_cast<f32x4*>(a.ws_o + (mpidx * G + hh) * D + d0) = acc * inv;
@@ -1194,7 +1402,7 @@ constexpr int kMergeWaves = 4;
 template <class TT, int D>
 __global__ void __launch_bounds__(64 * kMergeWaves)
 attn_merge_kernel(const AttnArgs a) {
-  using st = uint16_t;
+  using st = typename TT::storage;
   constexpr int CH = D / 8;
   const int G = a.G;
   const int wv = static_cast<int>(threadIdx.x >> 6), nwv = static_cast<int>(blockDim.x >> 6);
@@ -1262,7 +1470,7 @@ attn_merge_kernel(const AttnArgs a) {
       if (mmax != -INFINITY) {
 #pragma unroll
         for (int pp = 0; pp < kFew; ++pp) {
-          const float w = pp < total ? fast_exp2(lv[pp] - mmax) : 0.f;
+          const float w = pp < total ? TT::exp2(lv[pp] - mmax) : 0.f;
           lsum += w;
           acc0 += w * p0[pp];
           acc1 += w * p1[pp];
@@ -1295,13 +1503,13 @@ attn_merge_kernel(const AttnArgs a) {
         for (int k = 0; k < kBatch; ++k) bmax = fmaxf(bmax, lv[k]);
         if (bmax == -INFINITY) continue;
         const float mnew = fmaxf(mmax, bmax);
-        const float corr = fast_exp2(mmax - mnew);  // 0 while mmax is -inf
+        const float corr = TT::exp2(mmax - mnew);  // 0 while mmax is -inf
         lsum *= corr;
         acc0 *= corr;
         acc1 *= corr;
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) {
-          const float w = fast_exp2(lv[k] - mnew);
+          const float w = TT::exp2(lv[k] - mnew);
           lsum += w;
           acc0 += w * p0[k];
           acc1 += w * p1[k];
@@ -1324,7 +1532,7 @@ attn_merge_kernel(const AttnArgs a) {
           if (m2 != -INFINITY) {
             for (int w = 0; w < nwv; ++w) {
               const float* q = part_state[w][threadIdx.x];
-              const float c2 = fast_exp2(q[0] - m2);  // 0 for a wave that saw no part
+              const float c2 = TT::exp2(q[0] - m2);  // 0 for a wave that saw no part
               lsum += c2 * q[1];
               acc0 += c2 * f32x4{q[2], q[3], q[4], q[5]};
               acc1 += c2 * f32x4{q[6], q[7], q[8], q[9]};
@@ -1339,12 +1547,10 @@ attn_merge_kernel(const AttnArgs a) {
     const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
     const int h = kvh * G + hh;
     st* dp = static_cast<st*>(a.o) + t * a.o_st + static_cast<int64_t>(h) * a.o_sh + 8 * c;
-    *reinterpret_cast<u32x4*>(dp) =
-        u32x4{TT::pack2(acc0.x * inv, acc0.y * inv), TT::pack2(acc0.z * inv, acc0.w * inv),
-              TT::pack2(acc1.x * inv, acc1.y * inv), TT::pack2(acc1.z * inv, acc1.w * inv)};
+    TT::store8(dp, acc0 * inv, acc1 * inv);
     if (a.lse && c == 0)
       a.lse[t * a.l_st + static_cast<int64_t>(h) * a.l_sh] =
-          lsum > 0.f ? (mmax + __log2f(lsum)) * kLn2 : -INFINITY;
+          lsum > 0.f ? (mmax + TT::log2(lsum)) * kLn2 : -INFINITY;
   }
 }
 
@@ -1838,6 +2044,114 @@ attn_prefill_kernel(const AttnArgs a) {
   prefill_wg<TT, D, NM, SP>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
+// fp32 prefill: a work-group of kPre32Waves waves per (row, kv head, query
+// block of 16 NM / G queries); wave w takes the 16-key slices w, w +
+// kPre32Waves, ... straight from the paged cache into registers, the next
+// slice's loads in flight while one is computed, and the waves' states meet
+// in LDS.  Splitting the keys over the waves rather than the queries gives
+// short prompts enough waves: three prompts of 201 to 512 tokens (8 query
+// heads on 2 kv heads, D = 64) are 197 work-groups of 16 m-rows.  The MFMA
+// rate bounds it (a slice's K and V, 8 D * 16 bytes, feed D / 2 MFMAs of 32
+// cycles per 16 m-rows), so the caches' bandwidth is not what limits it and
+// tiles are not shared through LDS.  A 2048-token prompt (32 / 8 heads,
+// D = 128): 389 us, 88 TFLOP/s of the 154 a large fp32 matrix product
+// reaches, against 6.9 ms with one VALU wave per (query, head); the three
+// prompts above 112 -> 22.9 us a call.
+constexpr int kPre32Waves = 4;
+
+template <int D, int NM>
+__global__ void __launch_bounds__(64 * kPre32Waves)
+attn_prefill_f32_kernel(const AttnArgs a) {
+  using WA = WaveAttn<F32, D, NM, false>;
+  using Slice = typename WA::Slice;
+  constexpr int R = 16 * NM;  // m-rows
+  __shared__ __attribute__((aligned(16))) float so[kPre32Waves][R][D];
+  __shared__ float sm[kPre32Waves][R], sl[kPre32Waves][R];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int row = blockIdx.z;
+  const int kvh = static_cast<int>(blockIdx.x) % a.Hkv;
+  const int qblk = (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) / a.Hkv;  // longest first
+  const int qlen = a.q_lens[row];
+  const int Q = R / a.G;
+  const int q0 = qblk * Q;
+  if (qlen < 2 || q0 >= qlen) return;
+  const int nq = min(Q, qlen - q0);
+  const int off = a.q_offs[row], klen = a.k_lens[row];
+  const int64_t qs = a.q_starts[row];
+  const int bs = a.bs;
+  // Keys past the block table are not read.
+  const int64_t kmax = a.bt_stride * bs;
+  const int kend = static_cast<int>(
+      min(static_cast<int64_t>(max(a.causal ? min(klen, off + q0 + nq) : klen, 0)), kmax));
+  const int qpos_min = a.causal ? off + q0 : INT_MAX;
+  const int nsl = (kend + 15) / 16;
+
+  WA wa;
+  wa.setup(a, lane, kvh, qs, q0, nq, off);
+  const int32_t* btrow = a.bt + static_cast<int64_t>(row) * a.bt_stride;
+  const float* kbase = static_cast<const float*>(a.k) + static_cast<int64_t>(kvh) * a.k_sh;
+  const float* vbase = static_cast<const float*>(a.v) + static_cast<int64_t>(kvh) * a.v_sh;
+  auto load = [&](int i, Slice& T) {  // slice i, or nothing past the last
+    const bool live = i < nsl;
+    const int t = live ? 16 * i : 0;
+    int64_t id = live ? btrow[t / bs] : 0;
+    id = id < 0 ? 0 : (id >= a.num_blocks ? a.num_blocks - 1 : id);
+    wa.load_slice_from(a, kbase + id * a.k_sb, vbase + id * a.v_sb, t % bs, T, live);
+  };
+  if constexpr (WA::kLateV) {
+    Slice T;
+    for (int i = wave; i < nsl; i += kPre32Waves) {
+      load(i, T);
+      wa.compute_slice(a, 16 * i, kend, qpos_min, T);
+    }
+  } else {
+    Slice T0, T1;
+    if (wave < nsl) load(wave, T0);
+    for (int i = wave; i < nsl; i += 2 * kPre32Waves) {
+      load(i + kPre32Waves, T1);
+      wa.compute_slice(a, 16 * i, kend, qpos_min, T0);
+      if (i + kPre32Waves >= nsl) break;
+      load(i + 2 * kPre32Waves, T0);
+      wa.compute_slice(a, 16 * (i + kPre32Waves), kend, qpos_min, T1);
+    }
+  }
+  float lt[NM];
+  wa.row_sums(lt);
+#pragma unroll
+  for (int s = 0; s < NM; ++s) {
+    wa.store_row(so[wave][16 * s + wa.n], s, 1.f);
+    if (wa.g == 0) {
+      sm[wave][16 * s + wa.n] = wa.m[s];
+      sl[wave][16 * s + wa.n] = lt[s];
+    }
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < nq * a.G * (D / 4); it += 64 * kPre32Waves) {
+    const int r = it / (D / 4), d0 = 4 * (it % (D / 4));
+    const int64_t t = qs + q0 + r / a.G;
+    if (t >= a.total_q) break;  // (t does not fall as it grows)
+    float mx = sm[0][r];
+#pragma unroll
+    for (int w = 1; w < kPre32Waves; ++w) mx = fmaxf(mx, sm[w][r]);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    float lsum = 0.f;
+    if (mx != -INFINITY) {
+#pragma unroll
+      for (int w = 0; w < kPre32Waves; ++w) {
+        const float f = F32::exp2(sm[w][r] - mx);
+        lsum += f * sl[w][r];
+        acc += f * *reinterpret_cast<const f32x4*>(&so[w][r][d0]);
+      }
+    }
+    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    const int h = kvh * a.G + r % a.G;
+    F32::store4(static_cast<float*>(a.o) + t * a.o_st + static_cast<int64_t>(h) * a.o_sh + d0, acc * inv);
+    if (a.lse && d0 == 0)
+      a.lse[t * a.l_st + static_cast<int64_t>(h) * a.l_sh] = lsum > 0.f ? (mx + F32::log2(lsum)) * kLn2 : -INFINITY;
+  }
+}
+
 // ----------------------------------------------------------- VALU kernel --
 // One wave per (row, query, query head).  Lanes take 64 keys at a time for the
 // scores; for P.V each lane owns head_dim values lane, lane+64, ...
@@ -1952,6 +2266,10 @@ static int decode_waves(int64_t G, int64_t D) {
   return 8;
 }
 
+// fp32 rows of 256 values: K or V, Q and O take 64 registers each, and the
+// slice loop does not fit 256 (169 spilled), so 4 waves, one on each SIMD.
+constexpr int decode_waves_f32(int64_t D) { return D == 256 ? 4 : 8; }
+
 // LDS bytes a decode work-group of P ranges may use (see kMaxLdsBytes).
 static int64_t decode_lds_limit(int P, int64_t G, int64_t D) {
   return decode_lds_words(P, P, G, D) * 4 <= kMaxLdsBytes ? kMaxLdsBytes : kCuLdsBytes;
@@ -2017,7 +2335,7 @@ constexpr int prefill_nm(int64_t D) { return D == 64 ? 4 : (D == 128 || D == 96 
 // 16 m-rows; a prefill wave takes 16 NM / G whole queries, so a group that is
 // not a power of two leaves at most 2 of 32 m-rows empty for G <= 7).
 static bool mfma_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dtype) {
-  if (dtype != KVHOT_BF16 && dtype != KVHOT_F16) return false;
+  if (dtype_size(dtype) == 0) return false;
   if (D != 64 && D != 96 && D != 128 && D != 256) return false;
   return bs % 16 == 0 && Hq / Hkv <= 16;
 }
@@ -2029,11 +2347,14 @@ static bool mfma_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dt
 // per (query, head), 49.5 us here.
 static bool list_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dtype) {
   const int64_t G = Hq / Hkv;
-  return mfma_shape_ok(Hq, Hkv, D, bs, dtype) && D != 96 && (G & (G - 1)) == 0;
+  return mfma_shape_ok(Hq, Hkv, D, bs, dtype) && dtype != KVHOT_F32 && D != 96 && (G & (G - 1)) == 0;
 }
 
 // Queries of one (row, kv head) a prefill work-group takes.
 static int64_t prefill_queries(int64_t D, int64_t G) { return prefill_waves(D) * (16 * prefill_nm(D) / G); }
+
+// part_tokens of rows of up to max_k keys in one partition.
+static int whole_row_tokens(int64_t max_k) { return static_cast<int>(std::max<int64_t>((max_k + 15) / 16 * 16, 16)); }
 
 // Waves a grid launch without launch lists tries to fill: 8 on each CU.
 constexpr int64_t kGridWaves = 256 * 8;
@@ -2049,7 +2370,7 @@ static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
   Plan pl;
   pl.mfma = mfma_shape_ok(Hq, Hkv, D, bs, dtype);
   if (!pl.mfma || max_q < 1) return pl;
-  pl.waves = decode_waves(Hq / Hkv, D);
+  pl.waves = dtype == KVHOT_F32 ? decode_waves_f32(D) : decode_waves(Hq / Hkv, D);
   pl.lists = list_shape_ok(Hq, Hkv, D, bs, dtype);
   if (!pl.lists) {
     const int64_t slices = rows * Hkv * ((max_k + 15) / 16);
@@ -2057,6 +2378,9 @@ static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
         std::max<int64_t>(2, std::min<int64_t>(KVHOT_SLICES_PER_WAVE, slices / kGridWaves)));
   }
   pl.part_tokens = part_tokens > 0 ? static_cast<int>(part_tokens) : 16 * pl.waves * pl.wave_slices;
+  // partition_tokens cuts 16-bit rows; fp32 rows of a call that gives one are
+  // left whole.
+  if (dtype == KVHOT_F32 && part_tokens > 0) pl.part_tokens = whole_row_tokens(max_k);
   const int64_t parts = std::max<int64_t>((max_k + pl.part_tokens - 1) / pl.part_tokens, 1);
   if (parts > 65535) return pl;
   pl.grid_ok = true;
@@ -2542,8 +2866,8 @@ static void launch_decode(const AttnArgs& a, int64_t rows, int64_t n_dec, hipStr
   };
   // One instantiation per mode, so that the common one carries none of the
   // others' code.
-  if constexpr (SP) {
-    go(attn_decode_kernel<TT, D, W, false, false, true>);
+  if constexpr (SP || std::is_same<TT, F32>::value) {
+    go(attn_decode_kernel<TT, D, W, false, false, SP>);
   } else {
     const bool mr = da.dec_ranges > W, vb = a.verify && a.sched;
     if (mr && vb) go(attn_decode_kernel<TT, D, W, true, true>);
@@ -2557,8 +2881,9 @@ static void launch_decode(const AttnArgs& a, int64_t rows, int64_t n_dec, hipStr
 template <class TT, int D, bool SP>
 static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_q, int64_t n_dec,
                         int64_t n_pre, int64_t n_merge, int64_t n_pfx, hipStream_t stream) {
-  constexpr int NM = prefill_nm(D);
-  if constexpr (!SP)
+  constexpr bool F = std::is_same<TT, F32>::value;
+  constexpr int NM = F ? 1 : prefill_nm(D);
+  if constexpr (!SP && !F)
   if (a.sched && n_pfx > 0) {
     // Shared-prefix units, the first n_pfx of the prefill section, before
     // anything else on the caller's stream: the decode launch folds in the
@@ -2577,12 +2902,15 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
   const bool dec = !a.sched || n_dec > 0;
   const bool pre = a.sched ? n_pre > n_pfx : max_q >= 2;
   if (pre) {
-    const int64_t qpw = prefill_queries(D, a.G);
+    const int64_t qpw = F ? 16 * NM / a.G : prefill_queries(D, a.G);
     const int64_t nqb = (max_q + qpw - 1) / qpw;
     dim3 grid = a.sched ? dim3(static_cast<uint32_t>(n_pre - n_pfx))
                         : dim3(static_cast<uint32_t>(a.Hkv * nqb), 1u, static_cast<uint32_t>(rows));
     AttnArgs pa = a;
     if (a.sched) pa.sched = a.sched + 2 * (n_dec + n_pfx);
+    if constexpr (F)
+      hipLaunchKernelGGL((attn_prefill_f32_kernel<D, NM>), grid, dim3(64 * kPre32Waves), 0, stream, pa);
+    else
     hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM, SP>), grid, dim3(64 * prefill_waves(D)), 0, stream, pa);
   }
   if (dec) {
@@ -2597,7 +2925,7 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
 #else
     (void)waves;
 #endif
-    if (!launched) launch_decode<TT, D, 8, SP>(a, rows, n_dec, stream);
+    if (!launched) launch_decode<TT, D, F ? decode_waves_f32(D) : 8, SP>(a, rows, n_dec, stream);
   }
   if (a.sched ? n_merge > 0 : (!a.sched || n_dec > 0) && a.max_parts > 1) {
     dim3 mgrid = a.sched ? dim3(static_cast<uint32_t>(n_merge))
@@ -2808,7 +3136,7 @@ static int paged_attention_impl(
     const int64_t pb = partial_bytes(a.G, head_dim);
     if (!pl.lists && pl.partials > 0 && (!workspace || workspace_bytes < pl.workspace_bytes(a.G, head_dim))) {
       // Without room for partials every row is one partition.
-      pl.part_tokens = static_cast<int>(std::max<int64_t>((max_k_len + 15) / 16 * 16, 16));
+      pl.part_tokens = whole_row_tokens(max_k_len);
       pl.max_parts = 1;
       pl.partials = 0;
     }
@@ -2849,8 +3177,16 @@ static int paged_attention_impl(
       else KVHOT_MFMA(TT, 256, true);                                                 \
     }                                                                                 \
   } while (0)
-    if (dtype == KVHOT_BF16) KVHOT_MFMA_D(BF16);
-    else KVHOT_MFMA_D(F16);
+    if (dtype == KVHOT_F32) {
+      if (head_dim == 64) KVHOT_MFMA(F32, 64, false);
+      else if (head_dim == 96) KVHOT_MFMA(F32, 96, false);
+      else if (head_dim == 128) KVHOT_MFMA(F32, 128, false);
+      else KVHOT_MFMA(F32, 256, false);
+    } else if (dtype == KVHOT_BF16) {
+      KVHOT_MFMA_D(BF16);
+    } else {
+      KVHOT_MFMA_D(F16);
+    }
 #undef KVHOT_MFMA_D
 #undef KVHOT_MFMA
     return launch_status("paged_attention");
