@@ -168,7 +168,11 @@ int64_t kvhot_paged_attention_workspace_bytes(
  * metadata and first block, so the wave's first K/V loads depend on nothing
  * else; with KVHOT_VERIFY_BLOCKS in the attention call's attn_flags the
  * kernel checks that block against the device block table before using it), num_prefill_units per-work-group prefill units (longest
- * first), num_merge_units units, one per decode range cut into parts.
+ * first; a query block whose key range is long for a call that leaves the
+ * device idle is several units, each over part of its keys),
+ * num_merge_units units, one per decode range cut into parts or per few
+ * queries of prefill units cut by keys (their partials, with the decode
+ * rows' other ones, stay within KVHOT_NOALLOC_SCRATCH_BYTES).
  * Shared prefixes: when at least 4 decode rows (with causal masking or not)
  * read the same first 256 or more keys through the same physical blocks, the
  * keys of that common prefix are attended once, for all of those rows'
@@ -211,7 +215,8 @@ int64_t kvhot_paged_attention_schedule(
  * A query with no visible key gets out = 0 and lse = -inf.
  * Rows with n_q == 1 run the split-K flash-decoding kernel, plus a merge
  * launch when a decode row was split across work-groups; rows with
- * n_q >= 2 run the chunked-prefill kernel.  max_q_len / max_k_len must bound
+ * n_q >= 2 run the chunked-prefill kernel (and that merge launch where a
+ * schedule cut their units by keys).  max_q_len / max_k_len must bound
  * q_lens / k_lens (they size the grid; no device->host sync is made).
  * schedule: device copy of the units from kvhot_paged_attention_schedule for
  * exactly these lengths and sizes, with its four unit counts, the workspace

@@ -32,7 +32,9 @@
 //    (P^T keeps S^T's key order as the K dimension), and at head_dim <= 128
 //    the QK of the next tile runs beside the softmax of this one.  Causal
 //    mask from q_pos_offset; tiles past the work-group's last query are never
-//    loaded.
+//    loaded.  Units whose key range is long for a call that leaves the device
+//    idle are cut by keys (plan_prefill), their parts joined by
+//    attn_merge_kernel.
 //  * fp32: the decode kernel with WaveAttn<F32, ...> (v_mfma_f32_16x16x4_f32,
 //    operands straight from global memory) and attn_prefill_f32_kernel.
 //  * attn_generic_kernel<T>: VALU kernel for shapes the MFMA kernels do not
@@ -1391,30 +1393,95 @@ attn_decode_kernel(const AttnArgs a) {
   decode_wg<TT, D, W, MR, VB, SP>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// Combines the parts of split decode segments: (row, kv head) pieces that
-// ran in different work-groups and left (LSE, O) partials.  With a schedule,
-// work-group u takes merge unit u = (query token, kv head, parts, first
-// partial index), (first extra partial, extra partials) -- the extras are the
-// key splits of a shared prefix the row reads, written by prefix units --
-// each lane 8 head_dim values of one of the G query heads;
-// the kMergeWaves waves of the work-group fold a share of the parts each and
-// combine their states through LDS.  Without one, the grid is (head_dim
-// chunks, rows) of one-wave work-groups, and a row's parts are the fixed
-// partitions of part_tokens keys, recomputed as the decode kernel did.
+// Combines partials that ran in different work-groups.  With a schedule,
+// work-group u takes merge unit u, (query token, kv head, parts, first partial
+// index), (first extra partial, extra partials, queries, 0):
+//  * queries 0: a split decode segment's parts; the extras are the key splits
+//    of a shared prefix the row reads, written by prefix units.  Each lane
+//    takes 8 head_dim values of one of the G query heads; the kMergeWaves
+//    waves of the work-group fold a share of the parts each and combine their
+//    states through LDS.
+//  * queries n > 0: n consecutive queries of prefill units cut by keys, query
+//    i's parts from the first index + i * parts on; each thread takes 8
+//    head_dim values of one (query, head) (merge_queries sizes the unit).
+// Without one, the grid is (head_dim chunks, rows) of one-wave work-groups,
+// and a row's parts are the fixed partitions of part_tokens keys, recomputed
+// as the decode kernel did.
 constexpr int kMergeWaves = 4;
+
+// Queries of a merge unit of cut prefill units: one item per thread.
+__host__ __device__ constexpr int64_t merge_queries(int64_t G, int64_t D) {
+  return 64 * kMergeWaves / (G * (D / 8)) > 1 ? 64 * kMergeWaves / (G * (D / 8)) : 1;
+}
+
+// Running softmax state of 8 head_dim values.
+struct MergeState {
+  float mmax = -INFINITY, lsum = 0.f;
+  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+};
+
+// Folds inputs [lo, hi) into s, kBatch at a time: a batch's loads are issued
+// together, then folded in with the running max moved (long rows have tens of
+// parts, and a part-by-part loop waits for each load in turn).
+template <class TT, int D, class Input>
+__device__ inline void fold_parts(const AttnArgs& a, const Input& input, int lo, int hi, int hh, int c, MergeState& s) {
+  constexpr int kBatch = 8;
+  for (int b0 = lo; b0 < hi; b0 += kBatch) {
+    float lv[kBatch];
+    f32x4 p0[kBatch], p1[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      lv[k] = -INFINITY;
+      p0[k] = p1[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (b0 + k < hi) {
+        const int64_t pi = input(b0 + k);
+        lv[k] = a.ws_lse[pi * a.G + hh];
+        const f32x4* src = reinterpret_cast<const f32x4*>(a.ws_o + (pi * a.G + hh) * D + 8 * c);
+        p0[k] = src[0];
+        p1[k] = src[1];
+      }
+    }
+    float bmax = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) bmax = fmaxf(bmax, lv[k]);
+    if (bmax == -INFINITY) continue;
+    const float mnew = fmaxf(s.mmax, bmax);
+    const float corr = TT::exp2(s.mmax - mnew);  // 0 while mmax is -inf
+    s.lsum *= corr;
+    s.acc0 *= corr;
+    s.acc1 *= corr;
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) {
+      const float w = TT::exp2(lv[k] - mnew);
+      s.lsum += w;
+      s.acc0 += w * p0[k];
+      s.acc1 += w * p1[k];
+    }
+    s.mmax = mnew;
+  }
+}
+
+// Output and LSE of token t, query head h, head_dim chunk c.
+template <class TT>
+__device__ inline void store_merged(const AttnArgs& a, int64_t t, int h, int c, const MergeState& s) {
+  const float inv = s.lsum > 0.f ? 1.f / s.lsum : 0.f;
+  typename TT::storage* dp =
+      static_cast<typename TT::storage*>(a.o) + t * a.o_st + static_cast<int64_t>(h) * a.o_sh + 8 * c;
+  TT::store8(dp, s.acc0 * inv, s.acc1 * inv);
+  if (a.lse && c == 0)
+    a.lse[t * a.l_st + static_cast<int64_t>(h) * a.l_sh] =
+        s.lsum > 0.f ? (s.mmax + TT::log2(s.lsum)) * kLn2 : -INFINITY;
+}
 
 template <class TT, int D>
 __global__ void __launch_bounds__(64 * kMergeWaves)
 attn_merge_kernel(const AttnArgs a) {
-  using st = typename TT::storage;
   constexpr int CH = D / 8;
   const int G = a.G;
   const int wv = static_cast<int>(threadIdx.x >> 6), nwv = static_cast<int>(blockDim.x >> 6);
   int64_t t, base, xbase = 0;
-  int kvh, nparts, xparts = 0, it0, step;
+  int kvh, nparts, xparts = 0, queries = 0, it0, step;
   if (a.merge_units) {
-    // (query token, kv head, parts, first partial), (first extra partial,
-    // extra partials, 0, 0): the extra ones are a shared prefix's key splits.
     const int4 u = a.merge_units[2 * static_cast<int64_t>(blockIdx.x)];
     const int4 u1 = a.merge_units[2 * static_cast<int64_t>(blockIdx.x) + 1];
     t = u.x;
@@ -1423,6 +1490,7 @@ attn_merge_kernel(const AttnArgs a) {
     base = u.w;
     xbase = u1.x;
     xparts = u1.y;
+    queries = u1.z;
     it0 = threadIdx.x & 63;
     step = 64;
   } else {
@@ -1439,9 +1507,21 @@ attn_merge_kernel(const AttnArgs a) {
     it0 = idx - kvh * G * CH;  // (head in group, chunk) of this lane
     step = G * CH;             // one item per lane
   }
-  if (t < 0 || t >= a.total_q || kvh < 0 || kvh >= a.Hkv || nparts < 1 || base < 0 ||
-      base + nparts > a.num_partials || xparts < 0 || xbase < 0 || xbase + xparts > a.num_partials)
+  if (t < 0 || t >= a.total_q || kvh < 0 || kvh >= a.Hkv || nparts < 1 || base < 0 || queries < 0 ||
+      base + static_cast<int64_t>(max(queries, 1)) * nparts > a.num_partials || xparts < 0 || xbase < 0 ||
+      xbase + xparts > a.num_partials)
     return;
+  if (queries > 0) {
+    for (int it = threadIdx.x; it < queries * G * CH; it += 64 * kMergeWaves) {
+      const int i = it / (G * CH), hh = it % (G * CH) / CH, c = it % CH;
+      if (t + i >= a.total_q) break;
+      const int64_t first = base + static_cast<int64_t>(i) * nparts;
+      MergeState s;
+      fold_parts<TT, D>(a, [&](int p) -> int64_t { return first + p; }, 0, nparts, hh, c, s);
+      store_merged<TT>(a, t + i, kvh * G + hh, c, s);
+    }
+    return;
+  }
   // Partial of the i-th input: the parts, then the extra ones.
   const int total = nparts + xparts;
   auto input = [&](int i) -> int64_t { return i < nparts ? base + i : xbase + (i - nparts); };
@@ -1451,9 +1531,7 @@ attn_merge_kernel(const AttnArgs a) {
   for (int it = it0; it < G * CH; it += step) {
     const int hh = it / CH;
     const int c = it % CH;
-    float mmax = -INFINITY;
-    f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-    float lsum = 0.f;
+    MergeState s;
     if (total <= kFew) {
       float lv[kFew];
       f32x4 p0[kFew], p1[kFew];
@@ -1470,91 +1548,47 @@ attn_merge_kernel(const AttnArgs a) {
         }
       }
 #pragma unroll
-      for (int pp = 0; pp < kFew; ++pp) mmax = fmaxf(mmax, lv[pp]);
-      if (mmax != -INFINITY) {
+      for (int pp = 0; pp < kFew; ++pp) s.mmax = fmaxf(s.mmax, lv[pp]);
+      if (s.mmax != -INFINITY) {
 #pragma unroll
         for (int pp = 0; pp < kFew; ++pp) {
-          const float w = pp < total ? TT::exp2(lv[pp] - mmax) : 0.f;
-          lsum += w;
-          acc0 += w * p0[pp];
-          acc1 += w * p1[pp];
+          const float w = pp < total ? TT::exp2(lv[pp] - s.mmax) : 0.f;
+          s.lsum += w;
+          s.acc0 += w * p0[pp];
+          s.acc1 += w * p1[pp];
         }
       }
     } else {
-      // One pass, kBatch parts at a time: a batch's loads are issued
-      // together, then folded in with the running max moved (long rows have
-      // tens of parts, and a part-by-part loop waits for each load in turn).
-      constexpr int kBatch = 8;
       const int lo = static_cast<int>((static_cast<int64_t>(total) * wv) / nwv);
       const int hi = static_cast<int>((static_cast<int64_t>(total) * (wv + 1)) / nwv);
-      for (int b0 = lo; b0 < hi; b0 += kBatch) {
-        float lv[kBatch];
-        f32x4 p0[kBatch], p1[kBatch];
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          lv[k] = -INFINITY;
-          p0[k] = p1[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-          if (b0 + k < hi) {
-            const int64_t pi = input(b0 + k);
-            lv[k] = a.ws_lse[pi * G + hh];
-            const f32x4* src = reinterpret_cast<const f32x4*>(a.ws_o + (pi * G + hh) * D + 8 * c);
-            p0[k] = src[0];
-            p1[k] = src[1];
-          }
-        }
-        float bmax = -INFINITY;
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) bmax = fmaxf(bmax, lv[k]);
-        if (bmax == -INFINITY) continue;
-        const float mnew = fmaxf(mmax, bmax);
-        const float corr = TT::exp2(mmax - mnew);  // 0 while mmax is -inf
-        lsum *= corr;
-        acc0 *= corr;
-        acc1 *= corr;
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          const float w = TT::exp2(lv[k] - mnew);
-          lsum += w;
-          acc0 += w * p0[k];
-          acc1 += w * p1[k];
-        }
-        mmax = mnew;
-      }
+      fold_parts<TT, D>(a, input, lo, hi, hh, c, s);
       if (nwv > 1) {
         // The waves' states meet in LDS; wave 0 combines them.
         float* my = part_state[wv][threadIdx.x & 63];
-        my[0] = mmax;
-        my[1] = lsum;
-        my[2] = acc0.x; my[3] = acc0.y; my[4] = acc0.z; my[5] = acc0.w;
-        my[6] = acc1.x; my[7] = acc1.y; my[8] = acc1.z; my[9] = acc1.w;
+        my[0] = s.mmax;
+        my[1] = s.lsum;
+        my[2] = s.acc0.x; my[3] = s.acc0.y; my[4] = s.acc0.z; my[5] = s.acc0.w;
+        my[6] = s.acc1.x; my[7] = s.acc1.y; my[8] = s.acc1.z; my[9] = s.acc1.w;
         __syncthreads();
         if (wv == 0) {
-          float m2 = -INFINITY;
-          for (int w = 0; w < nwv; ++w) m2 = fmaxf(m2, part_state[w][threadIdx.x][0]);
-          lsum = 0.f;
-          acc0 = acc1 = f32x4{0.f, 0.f, 0.f, 0.f};
-          if (m2 != -INFINITY) {
+          MergeState m;
+          for (int w = 0; w < nwv; ++w) m.mmax = fmaxf(m.mmax, part_state[w][threadIdx.x][0]);
+          if (m.mmax != -INFINITY) {
             for (int w = 0; w < nwv; ++w) {
               const float* q = part_state[w][threadIdx.x];
-              const float c2 = TT::exp2(q[0] - m2);  // 0 for a wave that saw no part
-              lsum += c2 * q[1];
-              acc0 += c2 * f32x4{q[2], q[3], q[4], q[5]};
-              acc1 += c2 * f32x4{q[6], q[7], q[8], q[9]};
+              const float c2 = TT::exp2(q[0] - m.mmax);  // 0 for a wave that saw no part
+              m.lsum += c2 * q[1];
+              m.acc0 += c2 * f32x4{q[2], q[3], q[4], q[5]};
+              m.acc1 += c2 * f32x4{q[6], q[7], q[8], q[9]};
             }
           }
-          mmax = m2;
+          s = m;
         }
         __syncthreads();  // the states are read before the next item writes them
         if (wv > 0) continue;
       }
     }
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
-    const int h = kvh * G + hh;
-    st* dp = static_cast<st*>(a.o) + t * a.o_st + static_cast<int64_t>(h) * a.o_sh + 8 * c;
-    TT::store8(dp, acc0 * inv, acc1 * inv);
-    if (a.lse && c == 0)
-      a.lse[t * a.l_st + static_cast<int64_t>(h) * a.l_sh] =
-          lsum > 0.f ? (mmax + TT::log2(lsum)) * kLn2 : -INFINITY;
+    store_merged<TT>(a, t, kvh * G + hh, c, s);
   }
 }
 
@@ -1577,6 +1611,7 @@ attn_merge_kernel(const AttnArgs a) {
 // 8-wave work-group).  At head_dim 256 (a 128 KiB ring) one 8-wave
 // work-group takes the CU.
 constexpr int prefill_waves(int64_t D) { return D == 256 ? 8 : 4; }
+constexpr int prefill_groups_per_cu(int64_t D) { return D == 256 ? 1 : 2; }
 constexpr int kPreIssuers = 4;  // waves 0-3 issue the DMA, one per SIMD
 constexpr int kPreKeys = 32;
 // Interleave of the pipelined prefill phase: softmax VALU instructions
@@ -1688,11 +1723,14 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   // qt0 .. qt0 + nqg - 1, one per row) over keys [k0, kend_g) of the prefix
   // they share, read through `row`'s block table; every such key is visible
   // to every such query, and the normalised output of query i goes to the
-  // split-K partial pbase + i * pstride instead of the output.
-  int row, kvh, qblk = 0, k0 = 0, kend_g = 0, nqg = 0, off = 0, pbase = 0, pstride = 0;
+  // split-K partial pbase + i * pstride instead of the output.  A query block
+  // cut by keys is several units, second int4 (first key, -parts, partial of
+  // the first query, end key or INT_MAX): each attends its keys [k0, k1) and
+  // leaves partials with a stride of `parts`.
+  int row, kvh, qblk = 0, k0 = 0, kend_g = 0, nqg = 0, off = 0, pbase = 0, pstride = 0, k1 = INT_MAX;
   int64_t qs = 0;
   int q0g = 0;
-  bool prefix = false;
+  bool prefix = false, partial = false;  // partial: leaves split-K partials
   if (sched) {
     const int4 u = sched[2 * static_cast<int64_t>(bx)];
     const int4 u1 = sched[2 * static_cast<int64_t>(bx) + 1];
@@ -1708,7 +1746,14 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
       pstride = u1.w;
     } else {
       qblk = u.z;
+      if (u1.y < 0) {
+        k0 = u1.x;
+        pstride = -u1.y;
+        pbase = u1.z;
+        k1 = u1.w;
+      }
     }
+    partial = __builtin_amdgcn_readfirstlane(u1.y) != 0;
   } else {
     row = bz;
     kvh = bx % a.Hkv;
@@ -1717,14 +1762,14 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   row = __builtin_amdgcn_readfirstlane(row);
   kvh = __builtin_amdgcn_readfirstlane(kvh);
   qblk = __builtin_amdgcn_readfirstlane(qblk);
+  k0 = __builtin_amdgcn_readfirstlane(k0);
+  pbase = __builtin_amdgcn_readfirstlane(pbase);
+  pstride = __builtin_amdgcn_readfirstlane(pstride);
   if (row < 0 || kvh < 0 || kvh >= a.Hkv || qblk < 0) return;
   if (prefix) {
-    k0 = __builtin_amdgcn_readfirstlane(k0);
     kend_g = __builtin_amdgcn_readfirstlane(kend_g);
     qs = __builtin_amdgcn_readfirstlane(static_cast<int>(qs));
     nqg = __builtin_amdgcn_readfirstlane(nqg);
-    pbase = __builtin_amdgcn_readfirstlane(pbase);
-    pstride = __builtin_amdgcn_readfirstlane(pstride);
     if (k0 < 0 || k0 % kPreKeys != 0 || kend_g <= k0 || kend_g > a.k_lens[row] || qs < 0 || pbase < 0 ||
         pstride <= 0 || static_cast<int64_t>(pbase) + static_cast<int64_t>(nqg - 1) * pstride >= a.num_partials)
       return;
@@ -1739,9 +1784,15 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
     const int klen = a.k_lens[row];
     kend_g = max(a.causal ? min(klen, off + q0g + nqg) : klen, 0);
     qs = a.q_starts[row];
+    if (partial) {
+      if (k0 < 0 || k0 % kPreKeys != 0 || pbase < 0 ||
+          static_cast<int64_t>(pbase) + static_cast<int64_t>(nqg - 1) * pstride >= a.num_partials)
+        return;
+      kend_g = max(min(kend_g, __builtin_amdgcn_readfirstlane(k1)), k0);
+    }
   }
   const bool causal = a.causal && !prefix;
-  const int klen = prefix ? kend_g : a.k_lens[row];
+  const int klen = partial ? kend_g : a.k_lens[row];
   // This wave's queries and the keys they see.
   const int q0 = q0g + wave * QPW;
   const int nq = max(min(QPW, nqg - wave * QPW), 0);
@@ -2042,8 +2093,9 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
 #pragma unroll
   for (int s = 0; s < NM; ++s) {
     if (!wa.mval[s]) continue;
-    if (prefix)
-      wa.store_partial_blocks(a, s, static_cast<int64_t>(pbase) + static_cast<int64_t>(q0 + wa.row_query(a, s)) * pstride,
+    if (partial)  // (q0 counts from the row's first query, partials from the unit's)
+      wa.store_partial_blocks(a, s,
+                              static_cast<int64_t>(pbase) + static_cast<int64_t>(q0 - q0g + wa.row_query(a, s)) * pstride,
                               wa.row_head(a, s) - kvh * a.G, ltot[s]);
     else
       wa.store_final_blocks(a, s, qs + q0 + wa.row_query(a, s), ltot[s]);
@@ -2446,6 +2498,17 @@ static int64_t resident_decode_waves(int dtype, int64_t D, int W, int64_t G) {
   return static_cast<int64_t>(cus) * per * W;
 }
 
+// CUs of the current device (256 when no device can be queried).
+static int64_t device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) {
+    (void)hipGetLastError();
+    return 256;
+  }
+  return cus;
+}
+
 struct Piece {
   int row, kvh, s0, s1, part, seg;
 };
@@ -2835,31 +2898,124 @@ static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int3
   return true;
 }
 
-// Prefill launch list: (row, kv head, query block) units, longest key range first.
-static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int32_t* q_offs,
-                         int64_t rows, int64_t Hkv, int64_t G, int64_t D, bool causal,
-                         std::vector<int4>& pre) {
+// Prefill units of a call that leaves the device idle are cut by keys.  Such a
+// call ends with its longest unit: 225 queries on 1249 keys are 64 units of up
+// to 40 tiles, 42 us on 64 of 256 CUs.  A 32-key tile takes a work-group
+// tile_us: less with a CU to itself than beside another.  Parts end sooner but
+// cost a merge launch and a part's start (kSplitUs) and their fp32 partials'
+// way out and back (kSplitBytesPerUs, through the caches).  Of a few target
+// lengths from kMinSplitTiles and the even share per resident work-group
+// upwards, the one with the least estimate is taken if it is below kSplitGain
+// of the uncut call's.  Measured, uncut -> cut: 225 queries on 1249 keys (with
+// the call's 31 decode rows) 74.0 -> 57.4 us, 64 on 16448 391 -> 41, 3 on 8195
+// 251 -> 21.5, 300 on 4300 at head_dim 256 155 -> 48, a 2048-token prompt at
+// head_dim 64 64 -> 48.  Estimated to lose, and measured so with every unit
+// above 1.5 shares cut: two chunks of 512 on 2512 keys 66 -> 69, a 2048-token
+// prompt at head_dim 128 58.6 -> 60.2, 1024 tokens 31.7 -> 33.0; in a call that
+// fills the device (1024 units on 512 slots) 166 -> 173.
+constexpr int64_t kMinSplitTiles = 8;
+constexpr double kSplitUs = 9.0, kSplitBytesPerUs = 2e6, kSplitGain = 0.95;
+// Measured: 8192-token prompts (two work-groups on each CU; head_dim 256 has
+// one), and calls of one work-group per CU.
+constexpr double tile_us(int64_t D, bool alone) {
+  return D == 64 ? (alone ? 1.0 : 1.3) : D == 256 ? 1.15 : (alone ? 0.8 : 1.0);
+}
+// Most bytes of partials, those of the decode rows included: what the no-alloc
+// entry point holds.
+constexpr int64_t kMaxSplitBytes = KVHOT_NOALLOC_SCRATCH_BYTES;
+
+// Prefill launch list: (row, kv head, query block) units, longest key range
+// first; units cut by keys append their merge units to mrg and their partials
+// to `partials`.
+static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int32_t* q_offs, const int32_t* q_starts,
+                         int64_t rows, int64_t Hkv, int64_t G, int64_t D, bool causal, int64_t cus,
+                         std::vector<int4>& pre, std::vector<int4>& mrg, int64_t& partials) {
+  struct Unit {
+    int4 u, u1;
+    int64_t tiles;
+  };
+  const int64_t qpw = prefill_queries(D, G), slots = cus * prefill_groups_per_cu(D);
+  std::vector<Unit> units;
+  int64_t total = 0, longest = 0;
   for (int64_t r = 0; r < rows; ++r) {
     const int64_t qlen = q_lens[r], klen = k_lens[r], off = q_offs[r];
     if (qlen < 2) continue;
-    const int64_t qpw = prefill_queries(D, G);
     for (int64_t qb = 0; qb * qpw < qlen; ++qb) {
       const int64_t q0 = qb * qpw, nq = std::min(qpw, qlen - q0);
       const int64_t kend = std::max<int64_t>(causal ? std::min(klen, off + q0 + nq) : klen, 0);
+      const int64_t tiles = (kend + kPreKeys - 1) / kPreKeys;
       for (int64_t h = 0; h < Hkv; ++h)
-        pre.push_back(int4{static_cast<int>(r), static_cast<int>(h), static_cast<int>(qb),
-                           static_cast<int>((kend + kPreKeys - 1) / kPreKeys)});
+        units.push_back(Unit{int4{static_cast<int>(r), static_cast<int>(h), static_cast<int>(qb), static_cast<int>(tiles)},
+                             int4{0, 0, 0, 0}, tiles});
+      total += tiles * Hkv;
+      longest = std::max(longest, tiles);
     }
   }
-  std::stable_sort(pre.begin(), pre.end(), [](const int4& x, const int4& y) { return x.w > y.w; });
-  // Two int4 per work-group, like the decode descriptors (second one unused).
-  std::vector<int4> wide;
-  wide.reserve(2 * pre.size());
-  for (const int4& u : pre) {
-    wide.push_back(u);
-    wide.push_back(int4{0, 0, 0, 0});
+  // The target of least estimated time (0: no unit is cut).
+  int64_t target = 0;
+  const int64_t pb = partial_bytes(G, D), mq = merge_queries(G, D);
+  auto queries = [&](const Unit& un) { return std::min(qpw, q_lens[un.u.x] - un.u.z * qpw); };
+  auto parts_of = [](int64_t tiles, int64_t target_) {  // units up to half as long again stay whole
+    return 2 * tiles > 3 * target_ ? (tiles + target_ - 1) / target_ : 1;
+  };
+  const double share = static_cast<double>(total) / static_cast<double>(slots);
+  // Time per tile of n work-groups: between one on each CU and all slots taken.
+  auto per_tile = [&](int64_t n) {
+    const double f = std::min(1.0, std::max(0.0, static_cast<double>(n - cus) / static_cast<double>(cus)));
+    return tile_us(D, true) + f * (tile_us(D, false) - tile_us(D, true));
+  };
+  double best = kSplitGain * static_cast<double>(longest) * per_tile(static_cast<int64_t>(units.size()));
+  if (best > kSplitUs + std::max<double>(share, kMinSplitTiles) * tile_us(D, true)) {
+    int64_t last = 0;
+    for (double f : {1.25, 1.75, 2.5, 3.5, 5.0}) {
+      const int64_t t = std::max<int64_t>(kMinSplitTiles, static_cast<int64_t>(f * share));
+      if (t == last) continue;
+      last = t;
+      int64_t slowest = 0, bytes = 0, n = 0;
+      for (const Unit& un : units) {
+        const int64_t ks = parts_of(un.tiles, t);
+        n += ks;
+        slowest = std::max(slowest, (un.tiles + ks - 1) / ks);
+        if (ks > 1) bytes += ks * queries(un) * pb;
+      }
+      const double us =
+          static_cast<double>(slowest) * per_tile(n) + kSplitUs + static_cast<double>(bytes) / kSplitBytesPerUs;
+      if (us < best && bytes + partials * pb <= kMaxSplitBytes) {
+        best = us;
+        target = t;
+      }
+    }
   }
-  pre.swap(wide);
+  if (target > 0) {
+    const size_t whole = units.size();
+    for (size_t i = 0; i < whole; ++i) {
+      const Unit un = units[i];
+      const int64_t r = un.u.x, q0 = un.u.z * qpw, nq = queries(un), ks = parts_of(un.tiles, target);
+      if (ks == 1) continue;
+      for (int64_t k = 0; k < ks; ++k) {
+        const int64_t t0 = un.tiles * k / ks, t1 = un.tiles * (k + 1) / ks;
+        // (The last part's end comes from the lengths on the device.)
+        Unit part{un.u,
+                  int4{static_cast<int>(kPreKeys * t0), static_cast<int>(-ks), static_cast<int>(partials + k),
+                       k + 1 < ks ? static_cast<int>(kPreKeys * t1) : INT_MAX},
+                  t1 - t0};
+        part.u.w = static_cast<int>(part.tiles);
+        if (k == 0) units[i] = part;
+        else units.push_back(part);
+      }
+      for (int64_t q = 0; q < nq; q += mq) {
+        mrg.push_back(int4{static_cast<int>(q_starts[r] + q0 + q), un.u.y, static_cast<int>(ks),
+                           static_cast<int>(partials + q * ks)});
+        mrg.push_back(int4{0, 0, static_cast<int>(std::min(mq, nq - q)), 0});
+      }
+      partials += nq * ks;
+    }
+  }
+  std::stable_sort(units.begin(), units.end(), [](const Unit& x, const Unit& y) { return x.tiles > y.tiles; });
+  for (const Unit& un : units) {
+    pre.push_back(un.u);
+    pre.push_back(un.u1);
+  }
 }
 
 template <class TT, int D, int W, bool SP>
@@ -3007,7 +3163,8 @@ extern "C" int64_t kvhot_paged_attention_schedule(
     if (plan_decode(q_lens, k_lens, q_pos_offsets, q_starts, block_table, bt_row_stride, block_size,
                     num_rows, num_kv_heads, is_causal, pl.waves, ranges, groups, partition_tokens,
                     32 * head_dim * dtype_size(dtype), prefix_queries, dec, mrg, pfx, partials)) {
-      plan_prefill(q_lens, k_lens, q_pos_offsets, num_rows, num_kv_heads, G, head_dim, is_causal, pre);
+      plan_prefill(q_lens, k_lens, q_pos_offsets, q_starts, num_rows, num_kv_heads, G, head_dim, is_causal,
+                   device_cus(), pre, mrg, partials);
       pre.insert(pre.begin(), pfx.begin(), pfx.end());  // shared-prefix units first
     } else {  // counts beyond the descriptor fields: no schedule
       dec.clear();
