@@ -110,6 +110,26 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_NATIVE = None
+
+
+def native():
+    """kvhot_torch, the per-layer calls from torch tensors to the library of
+    load(); raises if it was not built."""
+    global _NATIVE
+    if _NATIVE is None:
+        lib = load()
+        try:
+            from . import kvhot_torch
+        except ImportError as e:
+            raise ImportError(f"kvhot_torch.so cannot be loaded ({e}): build it with "
+                              "`python serving-engine_amd/build.py`") from e
+        kvhot_torch.bind(*(ctypes.cast(getattr(lib, name), ctypes.c_void_p).value for name in (
+            "kvhot_paged_attention", "kvhot_paged_attention_workspace_bytes", "kvhot_reshape_and_cache")))
+        _NATIVE = kvhot_torch
+    return _NATIVE
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
         return _DTYPE_CODES[dtype]

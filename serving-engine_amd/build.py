@@ -1,9 +1,10 @@
-"""Builds libkvhot.so (the C-ABI HIP library) for gfx950 with hipcc.
+"""Builds libkvhot.so (the C-ABI HIP library) for gfx950 with hipcc, and
+kvhot_torch.so (the host side of the per-layer calls, against torch's headers).
 
 Usage: python serving-engine_amd/build.py [--jobs N] [--define NAME=VALUE ...]
 
-The library lands next to this file so it travels with the source tree.
-Sources compile in parallel to objects under _build/, then link into one
+The libraries land next to this file so they travel with the source tree.
+HIP sources compile in parallel to objects under _build/, then link into one
 shared object.  Always recompiles (the "does it build" check relies on that).
 """
 from __future__ import annotations
@@ -21,6 +22,8 @@ LIB_NAME = "libkvhot.so"
 LIB_PATH = os.path.join(HERE, LIB_NAME)
 BUILD_DIR = os.path.join(HERE, "_build")
 SOURCES = ["kvhot_cache.hip", "kvhot_attention.hip"]
+TORCH_SOURCE = "kvhot_torch.cpp"
+TORCH_PATH = os.path.join(HERE, "kvhot_torch.so")
 ARCH = "gfx950"
 
 
@@ -61,13 +64,36 @@ def _compile(src: str, obj: str, defines: list[str]) -> tuple[str, int, str]:
     return src, proc.returncode, out
 
 
+def _build_torch() -> tuple[str, int, str]:
+    """kvhot_torch.so: host code only, linked against the installed torch (and
+    given libkvhot's entry points when it is loaded)."""
+    import sysconfig
+
+    import torch
+
+    root = os.path.dirname(torch.__file__)
+    lib = os.path.join(root, "lib")
+    tmp = TORCH_PATH + ".tmp"
+    cmd = [hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           "-isystem", os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "include"),
+           "-isystem", os.path.join(root, "include"), "-isystem", sysconfig.get_paths()["include"],
+           os.path.join(CSRC, TORCH_SOURCE), "-o", tmp, f"-L{lib}", f"-Wl,-rpath,{lib}",
+           "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode == 0:
+        os.replace(tmp, TORCH_PATH)
+    return TORCH_SOURCE, proc.returncode, proc.stdout + proc.stderr
+
+
 def build(jobs: int | None = None, defines: list[str] | None = None, verbose: bool = False) -> str:
     defines = list(defines or [])
     os.makedirs(BUILD_DIR, exist_ok=True)
     objs = [os.path.join(BUILD_DIR, os.path.splitext(s)[0] + ".o") for s in SOURCES]
-    jobs = jobs or min(len(SOURCES), os.cpu_count() or 1)
+    jobs = jobs or min(len(SOURCES) + 1, os.cpu_count() or 1)
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as ex:
-        results = list(ex.map(lambda so: _compile(so[0], so[1], defines), zip(SOURCES, objs)))
+        host = ex.submit(_build_torch)
+        results = list(ex.map(lambda so: _compile(so[0], so[1], defines), zip(SOURCES, objs))) + [host.result()]
     failed = [(s, out) for s, rc, out in results if rc != 0]
     if verbose:
         for s, rc, out in results:

@@ -45,8 +45,9 @@
 #include <algorithm>
 #include <cfloat>
 #include <climits>
-#include <functional>
+#include <iterator>
 #include <mutex>
+#include <set>
 #include <type_traits>
 #include <vector>
 
@@ -2752,44 +2753,30 @@ static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int3
     }
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return n[x] > n[y]; });
     const int64_t ng = std::max<int64_t>(std::max<int64_t>(groups, 1), (nseg + W - 1) / W);
-    // Min-heap of (slices, work-group); a work-group leaves it when full.
-    std::vector<std::pair<int64_t, int64_t>> heap;
-    heap.reserve(ng);
-    for (int64_t g2 = 0; g2 < ng; ++g2) heap.emplace_back(0, g2);
+    // (slices, work-group) of the open work-groups, in order; one leaves when
+    // full.  (Looking at the first kMixCandidates in place: popping them off a
+    // heap and pushing all but one back took most of the planner's 1 ms for
+    // 256 rows.)
+    std::set<std::pair<int64_t, int64_t>> open;
+    for (int64_t g2 = 0; g2 < ng; ++g2) open.emplace_hint(open.end(), 0, g2);
     std::vector<std::vector<Piece>> lpt(ng);
     std::vector<int> held(static_cast<size_t>(ng * Hkv), 0);  // segments of each kv head per work-group
-    std::vector<std::pair<int64_t, int64_t>> cand;
     int64_t lmax = 0;
     for (int sg : order) {
       const int h = seg_kvh[sg];
-      cand.clear();
-      std::pop_heap(heap.begin(), heap.end(), std::greater<>());
-      cand.push_back(heap.back());
-      heap.pop_back();
-      while (static_cast<int>(cand.size()) < kMixCandidates && !heap.empty() &&
-             heap.front().first <= cand[0].first + kMixSlack) {
-        std::pop_heap(heap.begin(), heap.end(), std::greater<>());
-        cand.push_back(heap.back());
-        heap.pop_back();
-      }
-      size_t c = 0;
-      for (size_t k = 1; k < cand.size(); ++k)
-        if (held[cand[k].second * Hkv + h] < held[cand[c].second * Hkv + h]) c = k;
-      for (size_t k = 0; k < cand.size(); ++k) {
-        if (k == c) continue;
-        heap.push_back(cand[k]);
-        std::push_heap(heap.begin(), heap.end(), std::greater<>());
-      }
-      auto [ld, g2] = cand[c];
+      auto best = open.begin();
+      const int64_t most = best->first + kMixSlack;
+      int seen = 1;
+      for (auto it = std::next(best); it != open.end() && seen < kMixCandidates && it->first <= most; ++it, ++seen)
+        if (held[it->second * Hkv + h] < held[best->second * Hkv + h]) best = it;
+      auto node = open.extract(best);
+      auto& [ld, g2] = node.value();
       const int64_t s0 = pfx_sl[seg_row[sg]];
       lpt[g2].push_back(Piece{seg_row[sg], seg_kvh[sg], static_cast<int>(s0), static_cast<int>(s0 + n[sg]), 0, sg});
       ++held[g2 * Hkv + h];
       ld += n[sg];
       lmax = std::max(lmax, ld);
-      if (static_cast<int>(lpt[g2].size()) < W) {
-        heap.push_back({ld, g2});
-        std::push_heap(heap.begin(), heap.end(), std::greater<>());
-      }
+      if (static_cast<int>(lpt[g2].size()) < W) open.insert(std::move(node));
     }
     const double slice_us = static_cast<double>(slice_bytes) * ng / (kDecodeRateGBs * 1e3);
     if (!any_cut || static_cast<double>(lmax - target) * slice_us <= kMergeLaunchUs) {

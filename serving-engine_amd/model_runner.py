@@ -27,6 +27,7 @@ import torch
 
 from . import _lib
 from .block import BLOCK_SIZE
+from . import paged_attention_kernel as _attention
 from .paged_attention_kernel import build_paged_batch_metadata, paged_flash_attention
 from .request import RequestPhase
 
@@ -43,29 +44,6 @@ class _PagedKVCache:
         self.kv_cache = kv_cache
         self.num_kv_heads = kv_cache.shape[-2]
         self.head_dim = kv_cache.shape[-1]
-        self._pool = None      # the pool's launch constants, for write()
-        self._strides = {}     # ctypes stride arrays of key/value layouts seen by write()
-
-    def _pool_args(self):
-        """(pool, base pointer, layer and K/V byte strides, block/token/head/dim
-        strides as a ctypes array, block size, blocks, dtype, dtype code,
-        device index), computed once per pool tensor."""
-        kv = self.kv_cache
-        pool = self._pool
-        if pool is None or pool[0] is not kv:
-            st, es = kv.stride(), kv.element_size()
-            pool = (kv, kv.data_ptr(), st[0] * es, st[1] * es, _lib.i64_array(st[2:]), kv.shape[3], kv.shape[2],
-                    kv.dtype, _lib.dtype_code(kv.dtype), kv.get_device())
-            self._pool = pool
-        return pool
-
-    def _stride_array(self, strides):
-        arr = self._strides.get(strides)
-        if arr is None:
-            if len(self._strides) > 64:
-                self._strides.clear()
-            arr = self._strides[strides] = _lib.i64_array(strides)
-        return arr
 
     def write(self, key_states, value_states, layer_idx, write_index):
         """Scatter new K/V into their slots: k_cache.view(-1, Hkv, D)[write_index[i]] =
@@ -74,20 +52,24 @@ class _PagedKVCache:
         [1, Hkv, S, D]; write_index: int64 (or int32) [S] on the cache device.
         Slots outside the pool are skipped instead of raising.  (The launch
         reads the [S, Hkv, D] views' strides straight from the [1, Hkv, S, D]
-        tensors: an engine calls this once per layer per step.)"""
-        kv, base, layer_bytes, kv_bytes, cache_strides, bs, nblocks, dtype, code, dev = self._pool_args()
+        tensors: an engine calls this once per layer per step.  The ordinary
+        call runs in kvhot_torch; the rest here.)"""
+        kv = self.kv_cache
+        if _lib.native().append(kv, self.num_kv_heads, self.head_dim, key_states, value_states, layer_idx, write_index):
+            return
         shape = key_states.shape
         if len(shape) != 4 or shape[0] != 1 or value_states.shape != shape:
             raise ValueError(f"key {tuple(key_states.shape)} / value {tuple(value_states.shape)} must be [1, Hkv, S, D]")
         _, hkv, s, d = shape
         if hkv != self.num_kv_heads or d != self.head_dim:
             raise ValueError(f"key/value heads/dim {hkv}/{d} do not match the cache {self.num_kv_heads}/{self.head_dim}")
-        if key_states.dtype != dtype or value_states.dtype != dtype:
-            raise TypeError(f"key/value dtype {key_states.dtype} does not match the cache dtype {dtype}")
+        if key_states.dtype != kv.dtype or value_states.dtype != kv.dtype:
+            raise TypeError(f"key/value dtype {key_states.dtype} does not match the cache dtype {kv.dtype}")
         if write_index.dim() != 1 or write_index.shape[0] != s:
             raise ValueError(f"write_index must be [{s}], got {tuple(write_index.shape)}")
         if write_index.dtype is not torch.int64 and write_index.dtype is not torch.int32:
             raise TypeError(f"write_index must be int64 or int32, got {write_index.dtype}")
+        dev = kv.get_device()
         if key_states.get_device() != dev or value_states.get_device() != dev or write_index.get_device() != dev:
             raise ValueError("key, value, write_index and the cache must be on one GPU")
         if not 0 <= layer_idx < kv.shape[0]:
@@ -96,14 +78,15 @@ class _PagedKVCache:
             return
         if not write_index.is_contiguous():
             write_index = write_index.contiguous()
-        ks, vs = key_states.stride(), value_states.stride()
-        k_cache = base + layer_idx * layer_bytes
+        ks, vs, st, es = key_states.stride(), value_states.stride(), kv.stride(), kv.element_size()
+        cache_strides = _lib.i64_array(st[2:])
+        k_cache = kv.data_ptr() + layer_idx * st[0] * es
         status = _lib.load().kvhot_reshape_and_cache(
-            key_states.data_ptr(), self._stride_array((ks[2], ks[1], ks[3])),
-            value_states.data_ptr(), self._stride_array((vs[2], vs[1], vs[3])),
-            k_cache, cache_strides, k_cache + kv_bytes, cache_strides,
+            key_states.data_ptr(), _lib.i64_array((ks[2], ks[1], ks[3])),
+            value_states.data_ptr(), _lib.i64_array((vs[2], vs[1], vs[3])),
+            k_cache, cache_strides, k_cache + st[1] * es, cache_strides,
             write_index.data_ptr(), 1 if write_index.dtype is torch.int64 else 0,
-            s, hkv, d, bs, nblocks, code, _lib.stream_handle(kv.device))
+            s, hkv, d, kv.shape[3], kv.shape[2], _lib.dtype_code(kv.dtype), _lib.stream_handle(kv.device))
         if status:
             _lib.check(status, "kvhot_reshape_and_cache")
 
@@ -177,6 +160,14 @@ def hip_paged_attention_forward(module, query, key, value, attention_mask, scali
     query [1, Hq, S, D], key/value [1, Hkv, S, D]; kwargs cache, write_index,
     paged_metadata.  Returns ([1, S, Hq, D], None)."""
     cache: _PagedKVCache = kwargs["cache"]
+    if type(cache) is _PagedKVCache:
+        # Both launches from one native call (None: a call for the code below).
+        o = _lib.native().layer(
+            cache.kv_cache, cache.num_kv_heads, cache.head_dim, key, value, module.layer_idx, kwargs["write_index"],
+            query, kwargs["paged_metadata"], scaling, _attention.DEFAULT_PARTITION_TOKENS, _lib.KVHOT_CAUSAL,
+            _attention._WORKSPACES)
+        if o is not None:
+            return o, None
     cache.write(key, value, module.layer_idx, kwargs["write_index"])
     k_cache_blocks, v_cache_blocks = cache.blocks(module.layer_idx)
     q = query.transpose(1, 2).squeeze(0)  # [S, Hq, D]

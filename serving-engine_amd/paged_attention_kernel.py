@@ -41,6 +41,10 @@ PAGED_Q_TILE_SIZE = 16          # query rows per MFMA tile
 # Split-K partition size for decode rows; 0 lets the library choose.
 DEFAULT_PARTITION_TOKENS = 0
 
+# Units of a launch list planned in one call: 4096 decode ranges of a device-full
+# of work-groups (two on each of 256 CUs, 8 waves) and as many others.
+LIST_UNITS = 8192
+
 # Workspaces are per (device, stream): calls sharing one must be stream-ordered.
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 
@@ -86,17 +90,21 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
             host_bt.ctypes.data if host_bt.size else None, host_bt.shape[1] if host_bt.ndim == 2 else 0,
             len(host_q), hq, hkv, d, bs, pt, 1 if causal else 0, dtype)
     outs = tuple(ctypes.byref(c) for c in counts)
-    total = lib.kvhot_paged_attention_schedule(*args, None, 0, *outs)
+    # One call of the planner fills a list of up to LIST_UNITS units; a longer
+    # one takes a second call.
+    units = torch.empty((LIST_UNITS, 8), dtype=torch.int32, pin_memory=True)
+    total = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), LIST_UNITS, *outs)
     if total < 0:
         _lib.check(int(total), "kvhot_paged_attention_schedule")
     if total == 0:
         hit = None
     else:
-        units = torch.empty((total, 8), dtype=torch.int32, pin_memory=True)
-        got = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), total, *outs)
-        if got != total:
-            _lib.check(-1 if got >= 0 else int(got), "kvhot_paged_attention_schedule")
-        hit = (units.to(device, non_blocking=True),) + tuple(int(c.value) for c in counts)
+        if total > LIST_UNITS:
+            units = torch.empty((total, 8), dtype=torch.int32, pin_memory=True)
+            got = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), total, *outs)
+            if got != total:
+                _lib.check(-1 if got >= 0 else int(got), "kvhot_paged_attention_schedule")
+        hit = (units[:total].to(device, non_blocking=True),) + tuple(int(c.value) for c in counts)
     cache[key] = hit
     return hit
 
@@ -147,7 +155,17 @@ def paged_flash_attention(q, k_cache, v_cache, metadata, num_q_heads, num_kv_hea
     ``metadata["host_block_table"]``, against ``metadata["block_table"]``
     on the device, for callers that edit only the device copy (about 1-2%
     of a decode call).
+
+    The ordinary call runs in ``kvhot_torch``; what it does not take (a
+    step's first call of a shape, which builds the launch list, unusual
+    tensors, anything to refuse) is handled here.
     """
+    pt = DEFAULT_PARTITION_TOKENS if partition_tokens is None else int(partition_tokens)
+    flags = attn_flags(is_causal, deterministic, verify_block_table)
+    out = _lib.native().attention(q, k_cache, v_cache, metadata, num_q_heads, num_kv_heads, scale, bool(is_causal),
+                                  pt, flags, _WORKSPACES)
+    if out is not None:
+        return out
     if q.dim() != 3 or k_cache.dim() != 4 or v_cache.dim() != 4:
         raise ValueError("expected q [T, Hq, D] and k_cache/v_cache [N, block_size, Hkv, D]")
     total_query, hq, head_dim = q.shape
@@ -180,7 +198,6 @@ def paged_flash_attention(q, k_cache, v_cache, metadata, num_q_heads, num_kv_hea
     bt_stride = int(metadata.get("block_table_row_stride", bt.shape[1] if bt.dim() == 2 else 0))
     max_q = _host_max(metadata, "max_q_len", "q_lens")
     max_k = _host_max(metadata, "max_k_len", "k_lens")
-    pt = DEFAULT_PARTITION_TOKENS if partition_tokens is None else int(partition_tokens)
 
     lib = _lib.load()
     stream = _lib.stream_handle(device)
@@ -206,7 +223,7 @@ def paged_flash_attention(q, k_cache, v_cache, metadata, num_q_heads, num_kv_hea
         q_lens.data_ptr(), metadata["k_lens"].data_ptr(),
         metadata["q_starts"].data_ptr(), metadata["q_pos_offsets"].data_ptr(),
         num_rows, total_query, max_q, max_k, num_q_heads, num_kv_heads, head_dim,
-        block_size, num_blocks, float(scale), attn_flags(is_causal, deterministic, verify_block_table), dtype, pt,
+        block_size, num_blocks, float(scale), flags, dtype, pt,
         sched.data_ptr() if sched is not None else None, n_dec, n_pre, n_mrg, n_pfx,
         need if sched is not None else 0,
         ws.data_ptr() if ws is not None else None, ws.numel() if ws is not None else 0,
