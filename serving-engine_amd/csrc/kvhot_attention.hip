@@ -45,6 +45,7 @@
 #include <algorithm>
 #include <cfloat>
 #include <climits>
+#include <functional>
 #include <iterator>
 #include <mutex>
 #include <set>
@@ -2772,7 +2773,23 @@ static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int3
       if (static_cast<int>(lpt[g2].size()) < W) open.insert(std::move(node));
     }
     const double slice_us = static_cast<double>(slice_bytes) * ng / (kDecodeRateGBs * 1e3);
-    if (!any_cut || static_cast<double>(lmax - target) * slice_us <= kMergeLaunchUs) {
+    // Slices until the cut plan ends, its work-groups taken in order by
+    // `groups` resident ones.  (Work-groups that hold W short segments close
+    // early, so there may be more of them than that: 200 rows of 100 to 3000
+    // keys are 281, 640 slices at most and 1100 until the last one ends, where
+    // whole segments pack into 256 of up to 635; taken for balanced, the cut
+    // plan took 339 us, the packed one 205.)
+    int64_t cut_span = target;
+    if (any_cut && static_cast<int64_t>(wgs.size()) > groups) {
+      std::vector<int64_t> ends(std::max<int64_t>(groups, 1), 0);  // min-heap
+      for (const auto& wg : wgs) {
+        std::pop_heap(ends.begin(), ends.end(), std::greater<>());
+        for (const Piece& pc : wg) ends.back() += pc.s1 - pc.s0;
+        cut_span = std::max(cut_span, ends.back());
+        std::push_heap(ends.begin(), ends.end(), std::greater<>());
+      }
+    }
+    if (!any_cut || static_cast<double>(lmax - cut_span) * slice_us <= kMergeLaunchUs) {
       wgs.clear();
       for (auto& g2 : lpt)
         if (!g2.empty()) wgs.push_back(std::move(g2));
