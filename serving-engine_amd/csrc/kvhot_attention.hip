@@ -96,6 +96,10 @@ struct AttnArgs {
   int32_t fixed;
   // KVHOT_VERIFY_BLOCKS: decode waves check a launch list's first block.
   int32_t verify;
+  // attn_mixed_kernel: prefill units, decode work-groups, and the launch
+  // list's index of the first prefill unit.
+  int32_t mix_pre, mix_dec;
+  int64_t mix_first;
 };
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
@@ -830,12 +834,6 @@ struct WaveAttn<F32, D, NM, false> {
 // device-scope release per wave, which on gfx950 is an L2 write-back per wave
 // -- far slower than a launch.)
 
-// Slices in flight per decode wave: 1 (load the next slice after computing
-// this one) or 2 (double-buffered).
-#ifndef KVHOT_DECODE_DEPTH
-#define KVHOT_DECODE_DEPTH 1
-#endif
-
 #ifndef KVHOT_SLICES_PER_WAVE
 #define KVHOT_SLICES_PER_WAVE 8
 #endif
@@ -875,10 +873,13 @@ __device__ inline int wave_max_int(int x) {
 // partitions, decode_ranges); otherwise one range per wave, and P is W.
 // VB: KVHOT_VERIFY_BLOCKS (below).
 // SP: WaveAttn's.
-template <class TT, int D, int W, bool MR, bool VB, bool SP>
-__device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& a, const int4* sched, int bx, int by,
-                                                                int bz) {
-  extern __shared__ float smem[];
+// DEPTH: slices in flight per wave, 1 (load the next slice after computing this
+// one) or 2 (double-buffered; one range per wave, every block id from the
+// device table).  Two are slower where a CU holds 8 decode waves (54.3 against
+// 52.5 us on 64 rows of 128 to 2048 tokens); attn_mixed_kernel's 4 need them.
+template <class TT, int D, int W, bool MR, bool VB, bool SP, int DEPTH = 1>
+__device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& a, float* smem, const int4* sched,
+                                                                int bx, int by, int bz) {
   using st = typename TT::storage;
   // Wave-uniform values are pinned to SGPRs with readfirstlane: derived from
   // threadIdx they would otherwise count as divergent, putting block ids and
@@ -989,7 +990,6 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   Slice T;
   int i = s0;              // slice whose loads are in flight, if `have`
   bool have = nsl > 0;     // the first slice of the range is taken without a claim
-#if KVHOT_DECODE_DEPTH < 2
   // The first slice's block comes from the launch list, built from the host
   // copy of the block table, so that its loads wait for nothing.  With
   // KVHOT_VERIFY_BLOCKS the device table's entry is read before them and
@@ -1000,6 +1000,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   // (A buffer load: its wait is counted with the slice's vector loads, in
   // order, rather than with LDS operations.  The check is made once, before
   // the loop, so that nothing of it is carried through the loop.)
+  static_assert(DEPTH == 1 || (!MR && !VB), "two slices: one range per wave");
   const bool check_first = VB && sched && have && d_first >= 0;
   int dev_first = 0;
   if (check_first) {
@@ -1008,10 +1009,9 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
         block_rsrc(a.bt + static_cast<int64_t>(row) * a.bt_stride, static_cast<int>(4 * a.bt_stride));
     dev_first = __builtin_amdgcn_raw_buffer_load_b32(br, static_cast<int>(4 * lb), 0, 0);
   }
-  if (have)
+  if (DEPTH == 1 && have)
     wa.load_slice(a, kvh, d_first >= 0 ? min(static_cast<int64_t>(d_first), a.num_blocks - 1) : block_of(row, s0),
                   kb % bs, T);
-#endif
   if (lane == 0) {
     cnt[wave] = s0 + (have ? 1 : 0);
     dend[wave] = s0 + nsl;
@@ -1052,13 +1052,11 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   }
   // LDS-only barrier: the first slice's loads stay in flight across it.
   __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#if KVHOT_DECODE_DEPTH < 2
   if (check_first) {
     const int raw = __builtin_amdgcn_readfirstlane(dev_first);
     const int64_t want = raw < 0 ? 0 : (raw >= a.num_blocks ? a.num_blocks - 1 : raw);
     if (want != min(static_cast<int64_t>(d_first), a.num_blocks - 1)) wa.load_slice(a, kvh, want, kb % bs, T);
   }
-#endif
 
   // Claims one slice of range v (-1 when the range is used up).
   auto claim = [&](int v) -> int {
@@ -1099,7 +1097,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
     }
   };
 
-#if KVHOT_DECODE_DEPTH < 2
+  if constexpr (DEPTH == 1) {
   int cv = wave;           // range being claimed from
   int own = wave;          // the last of this wave's own ranges it entered (deterministic order)
   bool live = nsl > 0;     // the current segment may still have slices
@@ -1182,7 +1180,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
     cv = v;
     live = true;
   }
-#else
+  } else {
   // Two slices in flight per wave: the older in one buffer, the newer in the
   // other, and the block-table entry of the next claimed slice (iz) loading
   // behind them.  A half-step computes the older buffer, claims one more
@@ -1282,7 +1280,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
     half(T, ix, hx);
     if (!hx && !hy && !hz && !next_segment()) break;
   }
-#endif
+  }
   __syncthreads();
 
   // ---- merge: each range's slots are combined by the wave that set the
@@ -1392,7 +1390,8 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
 template <class TT, int D, int W, bool MR = false, bool VB = false, bool SP = false>
 __global__ void __launch_bounds__(64 * W)
 attn_decode_kernel(const AttnArgs a) {
-  decode_wg<TT, D, W, MR, VB, SP>(a, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
+  extern __shared__ float smem[];
+  decode_wg<TT, D, W, MR, VB, SP>(a, smem, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
 // Combines partials that ran in different work-groups.  With a schedule,
@@ -2104,6 +2103,45 @@ attn_prefill_kernel(const AttnArgs a) {
   prefill_wg<TT, D, NM, SP>(a, ring, a.sched, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
+// Prefill units and decode work-groups of one step in one launch (launch lists
+// without fixed partitions, head_dim 64 and 128): work-groups of 4 waves of
+// either kind, two to a CU, the decode ones with their state in the ring's
+// LDS.  The two kinds come in turns of kMixTurn work-groups (one per CU) while
+// both last, then the rest of the prefill units, then of the decode ones, so
+// that a CU tends to hold one of each, the one bound by the matrix cores, the
+// other by HBM.  The kernel's 256 registers leave two waves per SIMD, so a
+// decode wave keeps two slices in flight: with one slice, 512 decode work-groups
+// in the place of 256, 56 decode rows beside eight whole 512-token prompts
+// took 102 us, 86 as two launches, 76 with two slices.  Two launches -> one
+// (us): 64 decode rows beside 448 queries 78 -> 59, 200 rows beside 56 queries
+// 352 -> 217 (with the decode plan's own gain), 31 rows beside 225 queries on
+// 1249 keys 55.5 -> 48, 56 rows beside eight 512-token chunks on up to 4608
+// 267 -> 251, at head_dim 64 40 rows beside six chunks 104 -> 87.
+constexpr int kMixTurn = 256, kMixWaves = 4;
+template <class TT, int D, int NM>
+__global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_per_eu(2)))
+attn_mixed_kernel(const AttnArgs a) {
+  static_assert(prefill_waves(D) == kMixWaves, "one work-group size");
+  __shared__ __attribute__((aligned(16))) char ring[prefill_lds_bytes(D)];
+  const int bid = static_cast<int>(blockIdx.x);
+  const int turns = min(a.mix_pre, a.mix_dec) / kMixTurn;
+  bool pre;
+  int i;
+  if (bid < 2 * kMixTurn * turns) {
+    const int c = bid / kMixTurn;
+    pre = (c & 1) == 0;
+    i = kMixTurn * (c >> 1) + bid % kMixTurn;
+  } else {
+    i = bid - kMixTurn * turns;
+    pre = i < a.mix_pre;
+    if (!pre) i = bid - a.mix_pre;
+  }
+  if (pre)
+    prefill_wg<TT, D, NM, false>(a, ring, a.sched + 2 * a.mix_first, i, 0, 0);
+  else
+    decode_wg<TT, D, kMixWaves, false, false, false, 2>(a, reinterpret_cast<float*>(ring), a.sched, i, 0, 0);
+}
+
 // fp32 prefill: a work-group of kPre32Waves waves per (row, kv head, query
 // block of 16 NM / G queries); wave w takes the 16-key slices w, w +
 // kPre32Waves, ... straight from the paged cache into registers, the next
@@ -2343,8 +2381,8 @@ static int64_t decode_lds_limit(int P, int64_t G, int64_t D) {
 // a shared prefix -- a pool of 3W rather than W took the call from 75.1 to
 // 74.4 us, one box; P + 3W <= 64 keeps the merge's 64-lane ballot over the
 // slots.)
-static int decode_slots(int W, int P, int64_t G, int64_t D) {
-  const int64_t limit = decode_lds_limit(P, G, D);
+static int decode_slots(int W, int P, int64_t G, int64_t D, int64_t limit = 0) {
+  if (limit == 0) limit = decode_lds_limit(P, G, D);
   const int64_t base = decode_lds_words(P, P, G, D);
   if (base * 4 > limit) return 0;
   const int64_t spare = limit / 4 - base;
@@ -2364,7 +2402,7 @@ static int decode_slots(int W, int P, int64_t G, int64_t D) {
 constexpr int kFixedRangesPerWave = 4;
 static int decode_ranges(int W, int64_t G, int64_t D, bool fixed_partitions) {
   const int P = kFixedRangesPerWave * W;
-  if (!fixed_partitions || KVHOT_DECODE_DEPTH >= 2 || P + 3 * W > 64) return W;
+  if (!fixed_partitions || P + 3 * W > 64) return W;
   if (decode_slots(W, P, G, D) < P) return W;
   return P;
 }
@@ -2412,6 +2450,12 @@ static bool list_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dt
 
 // Queries of one (row, kv head) a prefill work-group takes.
 static int64_t prefill_queries(int64_t D, int64_t G) { return prefill_waves(D) * (16 * prefill_nm(D) / G); }
+
+// Whether a launch list's prefill units and decode work-groups run as one
+// launch (attn_mixed_kernel).
+static bool mixed_launch(int64_t D, bool fixed_partitions, bool has_decode, bool has_prefill) {
+  return D <= 128 && !fixed_partitions && has_decode && has_prefill;
+}
 
 // part_tokens of rows of up to max_k keys in one partition.
 static int whole_row_tokens(int64_t max_k) { return static_cast<int>(std::max<int64_t>((max_k + 15) / 16 * 16, 16)); }
@@ -2923,10 +2967,10 @@ constexpr int64_t kMaxSplitBytes = KVHOT_NOALLOC_SCRATCH_BYTES;
 
 // Prefill launch list: (row, kv head, query block) units, longest key range
 // first; units cut by keys append their merge units to mrg and their partials
-// to `partials`.
+// to `partials`.  others: the call's other partials.
 static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int32_t* q_offs, const int32_t* q_starts,
                          int64_t rows, int64_t Hkv, int64_t G, int64_t D, bool causal, int64_t cus,
-                         std::vector<int4>& pre, std::vector<int4>& mrg, int64_t& partials) {
+                         int64_t others, std::vector<int4>& pre, std::vector<int4>& mrg, int64_t& partials) {
   struct Unit {
     int4 u, u1;
     int64_t tiles;
@@ -2977,7 +3021,7 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
       }
       const double us =
           static_cast<double>(slowest) * per_tile(n) + kSplitUs + static_cast<double>(bytes) / kSplitBytesPerUs;
-      if (us < best && bytes + partials * pb <= kMaxSplitBytes) {
+      if (us < best && bytes + others * pb <= kMaxSplitBytes) {
         best = us;
         target = t;
       }
@@ -3013,6 +3057,27 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
     pre.push_back(un.u);
     pre.push_back(un.u1);
   }
+}
+
+// Decode work-groups of a mixed launch: as many as its slots leave free beside
+// the prefill units, about half at least, so that all start at once (one that
+// starts late ends late: the decode work is shared out equally); a sixteenth of
+// the slots stays free, since work-groups do not spread evenly enough to take
+// all (247 units and 265 decode work-groups on 512 slots 55.5 us, 254 of them
+// 48.0).  Where the prefill units take more than a round of the slots and as
+// long as the decode rows: all slots' worth of smaller ones, which then fill
+// the end of the launch too.  Measured with 256 / 512 decode work-groups (us):
+// 64 decode rows of 128 to 2048 beside 448 queries on 960 keys 59 / 72, 56
+// rows beside eight whole 512-token prompts 76 / 91; 4 rows of 20,000 to 30,000
+// beside two 1024-token chunks on up to 4000 156 / 145, 56 rows beside eight
+// 512-token chunks on up to 4608 (append included) 267 / 251.
+static int64_t mixed_decode_groups(int64_t D, int64_t cus, int64_t units, int64_t tiles, int64_t decode_bytes) {
+  const int64_t slots = cus * prefill_groups_per_cu(D);
+  const double pre_us = static_cast<double>(tiles) * tile_us(D, false) / static_cast<double>(slots);
+  const double dec_us = static_cast<double>(decode_bytes) / (kDecodeRateGBs * 1e3);
+  if (units >= slots && pre_us > 0.8 * dec_us) return slots;
+  if (units >= slots / 2) return slots / 2;
+  return std::max(slots / 2 - slots / 32, slots - slots / 16 - units);
 }
 
 template <class TT, int D, int W, bool SP>
@@ -3059,15 +3124,25 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
     hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM>), dim3(static_cast<uint32_t>(n_pfx)), dim3(64 * prefill_waves(D)), 0,
                        stream, xa);
   }
-  // Prefill units, then the decode work-groups, in launch order on the
-  // caller's stream.  (One launch holding both -- prefill units first,
-  // decode work-groups taking the CUs the prefill tail leaves idle -- needs
-  // one work-group size for both; with 8-wave prefill work-groups it saved
-  // 6 us on the mixed workload, less than two 4-wave prefill work-groups per
-  // CU save in the prefill alone.)
+  // Prefill units and decode work-groups: in one launch where the launch list
+  // was planned for it (kMixWaves waves), else one after the other.
   const bool dec = !a.sched || n_dec > 0;
   const bool pre = a.sched ? n_pre > n_pfx : max_q >= 2;
-  if (pre) {
+  bool mixed = false;
+  if constexpr (!SP && !F && D <= 128) {
+    if (a.sched && waves == kMixWaves) {
+      mixed = true;
+      AttnArgs ma = a;
+      ma.mix_pre = static_cast<int32_t>(n_pre - n_pfx);
+      ma.mix_dec = static_cast<int32_t>(n_dec / kMixWaves);
+      ma.mix_first = n_dec + n_pfx;
+      ma.dec_ranges = kMixWaves;
+      ma.dec_slots = decode_slots(kMixWaves, kMixWaves, a.G, D, prefill_lds_bytes(D));
+      const dim3 grid(static_cast<uint32_t>(ma.mix_pre) + static_cast<uint32_t>(ma.mix_dec));
+      hipLaunchKernelGGL((attn_mixed_kernel<TT, D, NM>), grid, dim3(64 * kMixWaves), 0, stream, ma);
+    }
+  }
+  if (pre && !mixed) {
     const int64_t qpw = F ? 16 * NM / a.G : prefill_queries(D, a.G);
     const int64_t nqb = (max_q + qpw - 1) / qpw;
     dim3 grid = a.sched ? dim3(static_cast<uint32_t>(n_pre - n_pfx))
@@ -3079,7 +3154,7 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
     else
     hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM, SP>), grid, dim3(64 * prefill_waves(D)), 0, stream, pa);
   }
-  if (dec) {
+  if (dec && !mixed) {
     bool launched = false;
 #if KVHOT_MAX_DECODE_WAVES >= 16
     if constexpr (D <= 128) {
@@ -3154,17 +3229,55 @@ extern "C" int64_t kvhot_paged_attention_schedule(
                             block_size, partition_tokens, dtype);
   if (pl.lists) {
     const int64_t G = num_q_heads / num_kv_heads;
-    const int64_t groups = resident_decode_waves(dtype, head_dim, pl.waves, G) / pl.waves;
+    const int64_t cus = device_cus();
+    // Prefill units, their partials numbered from 0 until the decode rows'
+    // count is known.
+    std::vector<int4> pmrg;
+    int64_t ppartials = 0;
+    auto prefill = [&](int64_t others) {
+      pre.clear();
+      pmrg.clear();
+      ppartials = 0;
+      plan_prefill(q_lens, k_lens, q_pos_offsets, q_starts, num_rows, num_kv_heads, G, head_dim, is_causal, cus, others,
+                   pre, pmrg, ppartials);
+    };
+    prefill(0);
+    int64_t keys = 0;  // of decode rows
+    bool has_decode = false;
+    for (int64_t r = 0; r < num_rows; ++r)
+      if (q_lens[r] == 1) {
+        has_decode = true;
+        keys += is_causal ? std::max(std::min(k_lens[r], q_pos_offsets[r] + 1), 0) : k_lens[r];
+      }
+    const bool mixed = mixed_launch(head_dim, partition_tokens > 0, has_decode, !pre.empty());
+    const int waves = mixed ? kMixWaves : pl.waves;
+    const int64_t slice_bytes = 32 * head_dim * dtype_size(dtype);
+    int64_t groups = 0;
+    if (mixed) {
+      int64_t tiles = 0;
+      for (size_t i = 0; i < pre.size(); i += 2) tiles += pre[i].w;
+      groups = mixed_decode_groups(head_dim, cus, static_cast<int64_t>(pre.size() / 2), tiles,
+                                   keys * num_kv_heads * slice_bytes / 16);
+    } else {
+      groups = resident_decode_waves(dtype, head_dim, pl.waves, G) / pl.waves;
+    }
     const int64_t prefix_queries = prefill_queries(head_dim, G);  // per prefill work-group
-    const int ranges = decode_ranges(pl.waves, G, head_dim, partition_tokens > 0);
+    const int ranges = decode_ranges(waves, G, head_dim, partition_tokens > 0);
     if (plan_decode(q_lens, k_lens, q_pos_offsets, q_starts, block_table, bt_row_stride, block_size,
-                    num_rows, num_kv_heads, is_causal, pl.waves, ranges, groups, partition_tokens,
-                    32 * head_dim * dtype_size(dtype), prefix_queries, dec, mrg, pfx, partials)) {
-      plan_prefill(q_lens, k_lens, q_pos_offsets, q_starts, num_rows, num_kv_heads, G, head_dim, is_causal,
-                   device_cus(), pre, mrg, partials);
+                    num_rows, num_kv_heads, is_causal, waves, ranges, groups, partition_tokens,
+                    slice_bytes, prefix_queries, dec, mrg, pfx, partials)) {
+      const int64_t room = kMaxSplitBytes / partial_bytes(G, head_dim);
+      if (ppartials > 0 && partials + ppartials > std::min<int64_t>(room, INT_MAX)) prefill(partials);
+      for (size_t i = 0; i < pre.size(); i += 2)
+        if (pre[i + 1].y < 0) pre[i + 1].z += static_cast<int>(partials);
+      for (size_t i = 0; i < pmrg.size(); i += 2) pmrg[i].w += static_cast<int>(partials);
+      mrg.insert(mrg.end(), pmrg.begin(), pmrg.end());
+      partials += ppartials;
       pre.insert(pre.begin(), pfx.begin(), pfx.end());  // shared-prefix units first
     } else {  // counts beyond the descriptor fields: no schedule
       dec.clear();
+      pre.clear();
+      pfx.clear();
       mrg.clear();
       partials = 0;
     }
@@ -3282,6 +3395,8 @@ static int paged_attention_impl(
     n_dec = n_pre = n_mrg = n_pfx = 0;
   }
   if (!schedule && !pl.grid_ok) pl.mfma = false;
+  const bool mixed = schedule && pl.lists && mixed_launch(head_dim, partition_tokens > 0, n_dec > 0, n_pre > n_pfx);
+  if (mixed) pl.waves = kMixWaves;
   if (schedule && pl.mfma && n_dec % pl.waves != 0)
     return set_error(KVHOT_EINVAL, "paged_attention: decode schedule is not whole work-groups");
   if (pl.mfma) {
