@@ -2118,7 +2118,7 @@ attn_prefill_kernel(const AttnArgs a) {
 // 1249 keys 55.5 -> 48, 56 rows beside eight 512-token chunks on up to 4608
 // 267 -> 251, at head_dim 64 40 rows beside six chunks 104 -> 87.
 constexpr int kMixTurn = 256, kMixWaves = 4;
-template <class TT, int D, int NM>
+template <class TT, int D, int NM, bool SP>
 __global__ void __launch_bounds__(64 * kMixWaves) __attribute__((amdgpu_waves_per_eu(2)))
 attn_mixed_kernel(const AttnArgs a) {
   static_assert(prefill_waves(D) == kMixWaves, "one work-group size");
@@ -2137,9 +2137,9 @@ attn_mixed_kernel(const AttnArgs a) {
     if (!pre) i = bid - a.mix_pre;
   }
   if (pre)
-    prefill_wg<TT, D, NM, false>(a, ring, a.sched + 2 * a.mix_first, i, 0, 0);
+    prefill_wg<TT, D, NM, SP>(a, ring, a.sched + 2 * a.mix_first, i, 0, 0);
   else
-    decode_wg<TT, D, kMixWaves, false, false, false, 2>(a, reinterpret_cast<float*>(ring), a.sched, i, 0, 0);
+    decode_wg<TT, D, kMixWaves, false, false, SP, 2>(a, reinterpret_cast<float*>(ring), a.sched, i, 0, 0);
 }
 
 // fp32 prefill: a work-group of kPre32Waves waves per (row, kv head, query
@@ -2413,6 +2413,8 @@ static int64_t partial_bytes(int64_t G, int64_t D) { return G * (D + 1) * 4; }
 struct Plan {
   bool mfma = false;     // the MFMA kernels take this shape
   bool lists = false;    // ... and launch lists are built for it
+  bool sp = false;       // ... by the kernels that split the probabilities
+  bool unsplit = false;  // unsplit_shape
   bool grid_ok = false;  // ... also without a schedule (partition count fits the grid)
   int waves = 0;         // waves per decode work-group
   int part_tokens = 0;   // keys per decode partition (no schedule)
@@ -2438,14 +2440,25 @@ static bool mfma_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dt
   return bs % 16 == 0 && Hq / Hkv <= 16;
 }
 
-// Shapes launch lists are built for; the others run from the grid, with
-// probabilities split in two (WaveAttn's SP), and without split-K when the
-// caller brings no workspace for it.  24 query heads on 8 kv heads, 13 decode
-// rows of up to 1500 keys and 5 chunks of up to 300: 925 us with one VALU wave
-// per (query, head), 49.5 us here.
-static bool list_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dtype) {
-  const int64_t G = Hq / Hkv;
-  return mfma_shape_ok(Hq, Hkv, D, bs, dtype) && dtype != KVHOT_F32 && D != 96 && (G & (G - 1)) == 0;
+// Shapes whose kernels split the probabilities in two (WaveAttn's SP): query
+// groups that are not a power of two, and head_dim 96.
+static bool split_probs(int64_t G, int64_t D) { return D == 96 || (G & (G - 1)) != 0; }
+
+// Calls launch lists are built for: the 16-bit shapes (fixed partitions of
+// those of split_probs run from the grid, which gives each its own
+// work-group).  Grid -> list for 24 / 8 heads at head_dim 128 (us): 64 rows of
+// 128 to 2048 keys 85 -> 48, 200 rows of 100 to 3000 295 -> 196, 128 rows behind
+// 1024 shared keys 158 -> 50, 56 rows beside eight 512-token prompts 130 -> 76,
+// 64 queries on 16448 keys 519 -> 41, 13 rows beside 5 chunks of up to 300
+// 48.3 -> 32.6.
+static bool list_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int64_t part_tokens, int dtype) {
+  return mfma_shape_ok(Hq, Hkv, D, bs, dtype) && dtype != KVHOT_F32 && (part_tokens == 0 || !split_probs(Hq / Hkv, D));
+}
+
+// Shapes whose decode rows run in one partition each where a call from the grid
+// has no room for their partials (fp32, and those of split_probs).
+static bool unsplit_shape(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dtype) {
+  return mfma_shape_ok(Hq, Hkv, D, bs, dtype) && (dtype == KVHOT_F32 || split_probs(Hq / Hkv, D));
 }
 
 // Queries of one (row, kv head) a prefill work-group takes.
@@ -2475,8 +2488,10 @@ static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
   pl.mfma = mfma_shape_ok(Hq, Hkv, D, bs, dtype);
   if (!pl.mfma || max_q < 1) return pl;
   pl.waves = dtype == KVHOT_F32 ? decode_waves_f32(D) : decode_waves(Hq / Hkv, D);
-  pl.lists = list_shape_ok(Hq, Hkv, D, bs, dtype);
-  if (!pl.lists) {
+  pl.lists = list_shape_ok(Hq, Hkv, D, bs, part_tokens, dtype);
+  pl.sp = dtype != KVHOT_F32 && split_probs(Hq / Hkv, D);
+  pl.unsplit = unsplit_shape(Hq, Hkv, D, bs, dtype);
+  if (pl.unsplit) {
     const int64_t slices = rows * Hkv * ((max_k + 15) / 16);
     pl.wave_slices = static_cast<int>(
         std::max<int64_t>(2, std::min<int64_t>(KVHOT_SLICES_PER_WAVE, slices / kGridWaves)));
@@ -2495,15 +2510,15 @@ static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
 
 // Decode work-groups the current device holds at once, times their waves
 // (one work-group on each of 256 CUs when no device can be queried).
-template <class TT, int D, int W>
+template <class TT, int D, int W, bool SP>
 static int decode_groups_per_cu(int64_t G) {
   int n = 0;
   const size_t lds = static_cast<size_t>(decode_lds_words(W, decode_slots(W, W, G, D), G, D) * 4);
-  if ((lds > kMaxLdsBytes &&
-       hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_decode_kernel<TT, D, W>),
-                           hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)) != hipSuccess) ||
-      hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, attn_decode_kernel<TT, D, W>, 64 * W, lds) !=
-          hipSuccess)
+  const auto kernel = attn_decode_kernel<TT, D, W, false, false, SP>;
+  if ((lds > kMaxLdsBytes && hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 static_cast<int>(lds)) != hipSuccess) ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, kernel, 64 * W, lds) != hipSuccess)
     n = 0;
   return n;
 }
@@ -2511,16 +2526,22 @@ static int decode_groups_per_cu(int64_t G) {
 template <class TT>
 static int decode_groups_per_cu(int64_t D, int W, int64_t G) {
 #if KVHOT_MAX_DECODE_WAVES >= 16
-  if (W == 16) {
-    if (D == 64) return decode_groups_per_cu<TT, 64, 16>(G);
-    return decode_groups_per_cu<TT, 128, 16>(G);
+  if (W == 16 && !split_probs(G, D)) {
+    if (D == 64) return decode_groups_per_cu<TT, 64, 16, false>(G);
+    return decode_groups_per_cu<TT, 128, 16, false>(G);
   }
 #else
   (void)W;
 #endif
-  if (D == 64) return decode_groups_per_cu<TT, 64, 8>(G);
-  if (D == 128) return decode_groups_per_cu<TT, 128, 8>(G);
-  return decode_groups_per_cu<TT, 256, 8>(G);
+  if (split_probs(G, D)) {
+    if (D == 64) return decode_groups_per_cu<TT, 64, 8, true>(G);
+    if (D == 96) return decode_groups_per_cu<TT, 96, 8, true>(G);
+    if (D == 128) return decode_groups_per_cu<TT, 128, 8, true>(G);
+    return decode_groups_per_cu<TT, 256, 8, true>(G);
+  }
+  if (D == 64) return decode_groups_per_cu<TT, 64, 8, false>(G);
+  if (D == 128) return decode_groups_per_cu<TT, 128, 8, false>(G);
+  return decode_groups_per_cu<TT, 256, 8, false>(G);
 }
 
 static int64_t resident_decode_waves(int dtype, int64_t D, int W, int64_t G) {
@@ -2958,7 +2979,9 @@ constexpr int64_t kMinSplitTiles = 8;
 constexpr double kSplitUs = 9.0, kSplitBytesPerUs = 2e6, kSplitGain = 0.95;
 // Measured: 8192-token prompts (two work-groups on each CU; head_dim 256 has
 // one), and calls of one work-group per CU.
-constexpr double tile_us(int64_t D, bool alone) {
+// (Split probabilities: 4096 tokens of 24 / 8 heads 157 us.)
+constexpr double tile_us(int64_t D, bool alone, bool sp = false) {
+  if (sp) return alone ? 1.0 : 1.5;
   return D == 64 ? (alone ? 1.0 : 1.3) : D == 256 ? 1.15 : (alone ? 0.8 : 1.0);
 }
 // Most bytes of partials, those of the decode rows included: what the no-alloc
@@ -3003,10 +3026,10 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
   // Time per tile of n work-groups: between one on each CU and all slots taken.
   auto per_tile = [&](int64_t n) {
     const double f = std::min(1.0, std::max(0.0, static_cast<double>(n - cus) / static_cast<double>(cus)));
-    return tile_us(D, true) + f * (tile_us(D, false) - tile_us(D, true));
+    return tile_us(D, true, split_probs(G, D)) + f * (tile_us(D, false, split_probs(G, D)) - tile_us(D, true, split_probs(G, D)));
   };
   double best = kSplitGain * static_cast<double>(longest) * per_tile(static_cast<int64_t>(units.size()));
-  if (best > kSplitUs + std::max<double>(share, kMinSplitTiles) * tile_us(D, true)) {
+  if (best > kSplitUs + std::max<double>(share, kMinSplitTiles) * tile_us(D, true, split_probs(G, D))) {
     int64_t last = 0;
     for (double f : {1.25, 1.75, 2.5, 3.5, 5.0}) {
       const int64_t t = std::max<int64_t>(kMinSplitTiles, static_cast<int64_t>(f * share));
@@ -3071,9 +3094,9 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
 // rows beside eight whole 512-token prompts 76 / 91; 4 rows of 20,000 to 30,000
 // beside two 1024-token chunks on up to 4000 156 / 145, 56 rows beside eight
 // 512-token chunks on up to 4608 (append included) 267 / 251.
-static int64_t mixed_decode_groups(int64_t D, int64_t cus, int64_t units, int64_t tiles, int64_t decode_bytes) {
+static int64_t mixed_decode_groups(int64_t D, int64_t G, int64_t cus, int64_t units, int64_t tiles, int64_t decode_bytes) {
   const int64_t slots = cus * prefill_groups_per_cu(D);
-  const double pre_us = static_cast<double>(tiles) * tile_us(D, false) / static_cast<double>(slots);
+  const double pre_us = static_cast<double>(tiles) * tile_us(D, false, split_probs(G, D)) / static_cast<double>(slots);
   const double dec_us = static_cast<double>(decode_bytes) / (kDecodeRateGBs * 1e3);
   if (units >= slots && pre_us > 0.8 * dec_us) return slots;
   if (units >= slots / 2) return slots / 2;
@@ -3108,20 +3131,19 @@ static void launch_decode(const AttnArgs& a, int64_t rows, int64_t n_dec, hipStr
   }
 }
 
-// SP: a shape without launch lists (a.sched null).
 template <class TT, int D, bool SP>
 static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_q, int64_t n_dec,
                         int64_t n_pre, int64_t n_merge, int64_t n_pfx, hipStream_t stream) {
   constexpr bool F = std::is_same<TT, F32>::value;
   constexpr int NM = F ? 1 : prefill_nm(D);
-  if constexpr (!SP && !F)
+  if constexpr (!F)
   if (a.sched && n_pfx > 0) {
     // Shared-prefix units, the first n_pfx of the prefill section, before
     // anything else on the caller's stream: the decode launch folds in the
     // partials they write.
     AttnArgs xa = a;
     xa.sched = a.sched + 2 * n_dec;
-    hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM>), dim3(static_cast<uint32_t>(n_pfx)), dim3(64 * prefill_waves(D)), 0,
+    hipLaunchKernelGGL((attn_prefill_kernel<TT, D, NM, SP>), dim3(static_cast<uint32_t>(n_pfx)), dim3(64 * prefill_waves(D)), 0,
                        stream, xa);
   }
   // Prefill units and decode work-groups: in one launch where the launch list
@@ -3129,7 +3151,7 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
   const bool dec = !a.sched || n_dec > 0;
   const bool pre = a.sched ? n_pre > n_pfx : max_q >= 2;
   bool mixed = false;
-  if constexpr (!SP && !F && D <= 128) {
+  if constexpr (!F && D <= 128) {
     if (a.sched && waves == kMixWaves) {
       mixed = true;
       AttnArgs ma = a;
@@ -3139,7 +3161,7 @@ static void launch_mfma(const AttnArgs& a, int waves, int64_t rows, int64_t max_
       ma.dec_ranges = kMixWaves;
       ma.dec_slots = decode_slots(kMixWaves, kMixWaves, a.G, D, prefill_lds_bytes(D));
       const dim3 grid(static_cast<uint32_t>(ma.mix_pre) + static_cast<uint32_t>(ma.mix_dec));
-      hipLaunchKernelGGL((attn_mixed_kernel<TT, D, NM>), grid, dim3(64 * kMixWaves), 0, stream, ma);
+      hipLaunchKernelGGL((attn_mixed_kernel<TT, D, NM, SP>), grid, dim3(64 * kMixWaves), 0, stream, ma);
     }
   }
   if (pre && !mixed) {
@@ -3256,7 +3278,7 @@ extern "C" int64_t kvhot_paged_attention_schedule(
     if (mixed) {
       int64_t tiles = 0;
       for (size_t i = 0; i < pre.size(); i += 2) tiles += pre[i].w;
-      groups = mixed_decode_groups(head_dim, cus, static_cast<int64_t>(pre.size() / 2), tiles,
+      groups = mixed_decode_groups(head_dim, G, cus, static_cast<int64_t>(pre.size() / 2), tiles,
                                    keys * num_kv_heads * slice_bytes / 16);
     } else {
       groups = resident_decode_waves(dtype, head_dim, pl.waves, G) / pl.waves;
@@ -3389,7 +3411,9 @@ static int paged_attention_impl(
 
   Plan pl = make_plan(num_rows, max_q_len, max_k_len, num_q_heads, num_kv_heads, head_dim,
                       block_size, partition_tokens, dtype);
-  if (!pl.lists) {  // a launch list means nothing for this shape
+  // A launch list means nothing for a shape without; the split-probability
+  // decode kernels have no form that checks its first blocks.
+  if (!pl.lists || (pl.sp && a.verify)) {
     schedule = nullptr;
     a.sched = a.merge_units = nullptr;
     n_dec = n_pre = n_mrg = n_pfx = 0;
@@ -3416,7 +3440,7 @@ static int paged_attention_impl(
   }
   if (pl.mfma) {
     const int64_t pb = partial_bytes(a.G, head_dim);
-    if (!pl.lists && pl.partials > 0 && (!workspace || workspace_bytes < pl.workspace_bytes(a.G, head_dim))) {
+    if (pl.unsplit && !schedule && pl.partials > 0 && (!workspace || workspace_bytes < pl.workspace_bytes(a.G, head_dim))) {
       // Without room for partials every row is one partition.
       pl.part_tokens = whole_row_tokens(max_k_len);
       pl.max_parts = 1;
@@ -3448,7 +3472,7 @@ static int paged_attention_impl(
   launch_mfma<TT, DD, SP>(a, pl.waves, num_rows, max_q_len, n_dec, n_pre, n_mrg, n_pfx, s)
 #define KVHOT_MFMA_D(TT)                                                              \
   do {                                                                                \
-    if (pl.lists) {                                                                   \
+    if (!pl.sp) {                                                                     \
       if (head_dim == 64) KVHOT_MFMA(TT, 64, false);                                  \
       else if (head_dim == 128) KVHOT_MFMA(TT, 128, false);                           \
       else KVHOT_MFMA(TT, 256, false);                                                \
@@ -3572,9 +3596,13 @@ extern "C" int kvhot_paged_attention_noalloc(
     need = kvhot_paged_attention_workspace_bytes(num_rows, total_query, max_q_len, max_k_len, num_q_heads,
                                                  num_kv_heads, head_dim, block_size, partition_tokens, dtype);
     if (need < 0) return set_error(static_cast<int>(need), "paged_attention_noalloc: bad sizes");
-    // (Shapes without launch lists run unsplit where their partials do not fit.)
-    if (need > KVHOT_NOALLOC_SCRATCH_BYTES && !list_shape_ok(num_q_heads, num_kv_heads, head_dim, block_size, dtype))
-      need = 0;
+  }
+  // (unsplit_shape runs from the grid, unsplit, where the partials do not fit.)
+  if (need > KVHOT_NOALLOC_SCRATCH_BYTES && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 &&
+      unsplit_shape(num_q_heads, num_kv_heads, head_dim, block_size, dtype)) {
+    schedule = nullptr;
+    num_decode_units = num_prefill_units = num_merge_units = num_prefix_units = schedule_workspace_bytes = 0;
+    need = 0;
   }
   if (need > KVHOT_NOALLOC_SCRATCH_BYTES)
     return set_error(KVHOT_EWORKSPACE, "paged_attention_noalloc: the call needs " + std::to_string(need) +

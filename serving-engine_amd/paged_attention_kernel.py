@@ -90,16 +90,17 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
             host_bt.ctypes.data if host_bt.size else None, host_bt.shape[1] if host_bt.ndim == 2 else 0,
             len(host_q), hq, hkv, d, bs, pt, 1 if causal else 0, dtype)
     outs = tuple(ctypes.byref(c) for c in counts)
-    # One call of the planner fills a list of up to LIST_UNITS units; a longer
-    # one takes a second call.
-    units = torch.empty((LIST_UNITS, 8), dtype=torch.int32, pin_memory=True)
-    total = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), LIST_UNITS, *outs)
+    # One call of the planner fills a list of as many units as the step's
+    # 16-token slices (up to LIST_UNITS); a longer one takes a second call.
+    room = min(LIST_UNITS, 256 + (int(host_k.sum()) // BLOCK_SIZE + len(host_k)) * hkv)
+    units = torch.empty((room, 8), dtype=torch.int32, pin_memory=True)
+    total = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), room, *outs)
     if total < 0:
         _lib.check(int(total), "kvhot_paged_attention_schedule")
     if total == 0:
         hit = None
     else:
-        if total > LIST_UNITS:
+        if total > room:
             units = torch.empty((total, 8), dtype=torch.int32, pin_memory=True)
             got = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), total, *outs)
             if got != total:

@@ -24,7 +24,7 @@ SPECS = {
 
 @pytest.mark.parametrize("hq,hkv,d,dtype", [
     (32, 8, 128, torch.bfloat16), (16, 1, 128, torch.float16), (8, 8, 128, torch.bfloat16), (16, 2, 64, torch.bfloat16),
-    (12, 12, 64, torch.float16),
+    (12, 12, 64, torch.float16), (24, 8, 128, torch.bfloat16), (12, 4, 96, torch.float16), (10, 2, 64, torch.bfloat16),
 ])
 @pytest.mark.parametrize("spec", list(SPECS))
 def test_mixed_launch(cuda, sea, wl, hq, hkv, d, dtype, spec):  # noqa: F811

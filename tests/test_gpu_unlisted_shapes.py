@@ -1,6 +1,6 @@
-"""Shapes that run the MFMA kernels from the padded grid, without launch
-lists: query groups of 1 to 16 heads that are not a power of two, and
-head_dim 96, against the fp64 oracle."""
+"""Shapes whose kernels split the probabilities in two -- query groups of 1 to
+16 heads that are not a power of two, and head_dim 96 -- from launch lists and
+from the padded grid, against the fp64 oracle."""
 import math
 
 import pytest
@@ -28,9 +28,13 @@ def test_grid_shapes(cuda, sea, wl, hq, hkv, d, dtype, layout):  # noqa: F811
     w = custom(wl, ROWS, hq, hkv, d, dtype)
     T = wl.make_tensors(w, cuda, layout=layout)
     ref_o, ref_l = oracle_step(w, T)
-    for pt in (None, 32, 512):
-        announce(f"grid shape Hq={hq} Hkv={hkv} D={d} {dtype} {layout} partition {pt}")
-        o, l = hip_step(sea, wl, w, T, partition_tokens=pt)
+    listed = wl.metadata_tensors(w, cuda)
+    grid = {k: v for k, v in listed.items() if not k.startswith("host_")}
+    for pt, meta in ((p, m) for p in (None, 32, 512) for m in (listed, grid)):
+        announce(f"shape Hq={hq} Hkv={hkv} D={d} {dtype} {layout} partition {pt}, {'list' if meta is listed else 'grid'}")
+        o, l = hip_step(sea, wl, w, T, partition_tokens=pt, meta=meta)
+        if meta is listed and pt is None:
+            assert all(plan[1] > 0 and plan[2] > 0 for plan in meta["_schedules"].values())
         assert_attention(w, o, l, ref_o, ref_l, rows=[i for i, x in enumerate(w.rows) if x.q_len > 0])
 
 

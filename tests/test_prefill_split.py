@@ -64,7 +64,7 @@ ROWS = [
 @pytest.mark.gpu
 @pytest.mark.parametrize("hq,hkv,d,dtype", [
     (32, 8, 128, torch.bfloat16), (12, 12, 64, torch.float16), (8, 2, 64, torch.bfloat16), (16, 4, 256, torch.bfloat16),
-    (16, 1, 128, torch.float16),
+    (16, 1, 128, torch.float16), (24, 8, 128, torch.bfloat16), (12, 4, 96, torch.float16),
 ])
 def test_cut_units(cuda, sea, wl, hq, hkv, d, dtype):  # noqa: F811
     for spec in ROWS:
