@@ -35,6 +35,8 @@
 //    loaded.  Units whose key range is long for a call that leaves the device
 //    idle are cut by keys (plan_prefill), their parts joined by
 //    attn_merge_kernel.
+//  * attn_mixed_kernel<T, D, NM, SP>: a step's prefill units and decode
+//    work-groups in one launch, 4 waves each (head_dim 64 to 128).
 //  * fp32: the decode kernel with WaveAttn<F32, ...> (v_mfma_f32_16x16x4_f32,
 //    operands straight from global memory) and attn_prefill_f32_kernel.
 //  * attn_generic_kernel<T>: VALU kernel for shapes the MFMA kernels do not
@@ -3419,7 +3421,10 @@ static int paged_attention_impl(
     n_dec = n_pre = n_mrg = n_pfx = 0;
   }
   if (!schedule && !pl.grid_ok) pl.mfma = false;
-  const bool mixed = schedule && pl.lists && mixed_launch(head_dim, partition_tokens > 0, n_dec > 0, n_pre > n_pfx);
+  // (A list planned without partition_tokens is taken as such where another
+  // value is passed here and its work-groups are of kMixWaves.)
+  const bool mixed = schedule && pl.lists &&
+                     mixed_launch(head_dim, partition_tokens > 0 && n_dec % pl.waves == 0, n_dec > 0, n_pre > n_pfx);
   if (mixed) pl.waves = kMixWaves;
   if (schedule && pl.mfma && n_dec % pl.waves != 0)
     return set_error(KVHOT_EINVAL, "paged_attention: decode schedule is not whole work-groups");

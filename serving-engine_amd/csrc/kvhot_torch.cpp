@@ -13,7 +13,7 @@
 // MI355X: an append of 16 tokens 8.2 -> 4.3 us, attention of one row of 1001
 // keys 20.2 -> 12.1, a layer (append and attention) of 8 decode rows 33 -> 16,
 // of 4 short fp32 rows 31.5 -> 12.2, 16 layers of 16 rows with their step's
-// metadata and launch list 770 -> 410.  From here on the GPU's own time bounds
+// metadata and launch list 770 -> 360 to 450.  From here on the GPU's own time bounds
 // all of these but the last two.
 #include <Python.h>
 

@@ -90,22 +90,23 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
             host_bt.ctypes.data if host_bt.size else None, host_bt.shape[1] if host_bt.ndim == 2 else 0,
             len(host_q), hq, hkv, d, bs, pt, 1 if causal else 0, dtype)
     outs = tuple(ctypes.byref(c) for c in counts)
-    # One call of the planner fills a list of as many units as the step's
-    # 16-token slices (up to LIST_UNITS); a longer one takes a second call.
-    room = min(LIST_UNITS, 256 + (int(host_k.sum()) // BLOCK_SIZE + len(host_k)) * hkv)
-    units = torch.empty((room, 8), dtype=torch.int32, pin_memory=True)
-    total = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), room, *outs)
+    # One call of the planner fills a list of as many units as the step has
+    # 16-token slices at most (up to LIST_UNITS); a longer one takes a second.
+    room = min(LIST_UNITS, 256 + (_host_max(metadata, "max_k_len", "k_lens") // BLOCK_SIZE + 1) * len(host_q) * hkv)
+    units = np.empty((room, 8), dtype=np.int32)
+    total = int(lib.kvhot_paged_attention_schedule(*args, units.ctypes.data, room, *outs))
+    if total > room:
+        units = np.empty((total, 8), dtype=np.int32)
+        if lib.kvhot_paged_attention_schedule(*args, units.ctypes.data, total, *outs) != total:
+            total = -1
     if total < 0:
-        _lib.check(int(total), "kvhot_paged_attention_schedule")
+        _lib.check(total, "kvhot_paged_attention_schedule")
     if total == 0:
         hit = None
     else:
-        if total > room:
-            units = torch.empty((total, 8), dtype=torch.int32, pin_memory=True)
-            got = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), total, *outs)
-            if got != total:
-                _lib.check(-1 if got >= 0 else int(got), "kvhot_paged_attention_schedule")
-        hit = (units[:total].to(device, non_blocking=True),) + tuple(int(c.value) for c in counts)
+        staged = torch.empty((total, 8), dtype=torch.int32, pin_memory=True)
+        staged.numpy()[:] = units[:total]
+        hit = (staged.to(device, non_blocking=True),) + tuple(int(c.value) for c in counts)
     cache[key] = hit
     return hit
 
