@@ -134,10 +134,14 @@ __device__ inline rsrc_words_t rsrc_words(const void* base, int bytes) {
 // compiler's own vmcnt waits stay correct: DMAs it does not know of only make
 // them wait longer.)  It sets M0, which the compiler treats as reserved and
 // does not track across asm: a kernel that uses it may hold nothing of its
-// own in M0 (the prefill kernel uses M0 for these DMAs only).
+// own in M0 (the prefill and mixed kernels use M0 for these DMAs only).  An
+// LDS DMA may read M0 one wait state after a scalar write of it at the
+// earliest; the compiler's hazard pass keeps that distance for its own
+// instructions and does not look inside asm, hence the s_nop.
 __device__ inline void dma16_asm(rsrc_words_t r, void* dst, int off) {
   const uint32_t lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)dst));
-  asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off), "s"(r)
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(off),
+               "s"(r)
                : "memory");
 }
 
