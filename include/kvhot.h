@@ -164,7 +164,8 @@ int64_t kvhot_paged_attention_workspace_bytes(
  * work-group, one device-full of work-groups; a range cut in two becomes
  * "parts" in different work-groups.  Units of 8 int32, in order:
  * num_decode_units range descriptors (whole work-groups, of 8 waves, or of 4
- * where prefill units share their launch: one per wave, or
+ * where prefill units share their launch, then an odd number of work-groups,
+ * by which the attention call tells them: one per wave, or
  * with partition_tokens > 0 up to four per wave; each carries its row's
  * metadata and first block, so the wave's first K/V loads depend on nothing
  * else; with KVHOT_VERIFY_BLOCKS in the attention call's attn_flags the

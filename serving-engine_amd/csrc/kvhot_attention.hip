@@ -2470,11 +2470,17 @@ static bool unsplit_shape(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dt
 // Queries of one (row, kv head) a prefill work-group takes.
 static int64_t prefill_queries(int64_t D, int64_t G) { return prefill_waves(D) * (16 * prefill_nm(D) / G); }
 
-// Whether a launch list's prefill units and decode work-groups run as one
-// launch (attn_mixed_kernel).
+// Whether the planner lays a call's prefill units and decode work-groups out
+// for one launch (attn_mixed_kernel).
 static bool mixed_launch(int64_t D, bool fixed_partitions, bool has_decode, bool has_prefill) {
   return D <= 128 && !fixed_partitions && has_decode && has_prefill;
 }
+
+// Whether a launch list of n_dec decode descriptors was laid out so.  The list
+// itself says it, whatever partition_tokens its call is passed: work-groups of
+// kMixWaves descriptors are padded to an odd number of them, other lists are
+// whole work-groups of at least twice as many.
+static bool is_mixed_list(int64_t n_dec) { return n_dec % (2 * kMixWaves) == kMixWaves; }
 
 // part_tokens of rows of up to max_k keys in one partition.
 static int whole_row_tokens(int64_t max_k) { return static_cast<int>(std::max<int64_t>((max_k + 15) / 16 * 16, 16)); }
@@ -3294,6 +3300,11 @@ extern "C" int64_t kvhot_paged_attention_schedule(
     if (plan_decode(q_lens, k_lens, q_pos_offsets, q_starts, block_table, bt_row_stride, block_size,
                     num_rows, num_kv_heads, is_causal, waves, ranges, groups, partition_tokens,
                     slice_bytes, prefix_queries, dec, mrg, pfx, partials)) {
+      if (mixed && !is_mixed_list(static_cast<int64_t>(dec.size() / 2)))
+        for (int e = 0; e < kMixWaves; ++e) {  // an empty work-group
+          dec.push_back(int4{-1, 0, 0, 0});
+          dec.push_back(int4{0, 0, -1, 0});
+        }
       const int64_t room = kMaxSplitBytes / partial_bytes(G, head_dim);
       if (ppartials > 0 && partials + ppartials > std::min<int64_t>(room, INT_MAX)) prefill(partials);
       for (size_t i = 0; i < pre.size(); i += 2)
@@ -3425,11 +3436,7 @@ static int paged_attention_impl(
     n_dec = n_pre = n_mrg = n_pfx = 0;
   }
   if (!schedule && !pl.grid_ok) pl.mfma = false;
-  // (A list planned without partition_tokens is taken as such where another
-  // value is passed here and its work-groups are of kMixWaves.)
-  const bool mixed = schedule && pl.lists &&
-                     mixed_launch(head_dim, partition_tokens > 0 && n_dec % pl.waves == 0, n_dec > 0, n_pre > n_pfx);
-  if (mixed) pl.waves = kMixWaves;
+  if (schedule && head_dim <= 128 && is_mixed_list(n_dec)) pl.waves = kMixWaves;
   if (schedule && pl.mfma && n_dec % pl.waves != 0)
     return set_error(KVHOT_EINVAL, "paged_attention: decode schedule is not whole work-groups");
   if (pl.mfma) {
@@ -3473,9 +3480,10 @@ static int paged_attention_impl(
       a.wave_slices = pl.wave_slices;
     }
     // A launch list of fixed partitions groups its decode ranges as the
-    // planner did (the same partition_tokens is passed to both calls; with
-    // another value the ranges come in groups of one per wave, which gives
-    // the same results).
+    // planner did where the call is passed partition_tokens too.  Passed
+    // another value than was planned with, ranges are grouped by whole planned
+    // work-groups (launch_decode) or by W of one, which hold whole segments
+    // too: the results are the same.
     a.dec_ranges = schedule ? decode_ranges(pl.waves, a.G, head_dim, partition_tokens > 0) : pl.waves;
 #define KVHOT_MFMA(TT, DD, SP) \
   launch_mfma<TT, DD, SP>(a, pl.waves, num_rows, max_q_len, n_dec, n_pre, n_mrg, n_pfx, s)
