@@ -3428,9 +3428,11 @@ static int paged_attention_impl(
 
   Plan pl = make_plan(num_rows, max_q_len, max_k_len, num_q_heads, num_kv_heads, head_dim,
                       block_size, partition_tokens, dtype);
-  // A launch list means nothing for a shape without; the split-probability
-  // decode kernels have no form that checks its first blocks.
-  if (!pl.lists || (pl.sp && a.verify)) {
+  // A launch list means nothing for a shape without (also one of no units: what
+  // the planner gives such a shape, or one of split_probs with fixed partitions);
+  // the split-probability decode kernels have no form that checks its first
+  // blocks.
+  if (!pl.lists || (pl.sp && (a.verify || n_dec + n_pre == 0))) {
     schedule = nullptr;
     a.sched = a.merge_units = nullptr;
     n_dec = n_pre = n_mrg = n_pfx = 0;
