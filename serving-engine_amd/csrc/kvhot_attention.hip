@@ -3437,6 +3437,8 @@ static int paged_attention_impl(
     a.sched = a.merge_units = nullptr;
     n_dec = n_pre = n_mrg = n_pfx = 0;
   }
+  // fp32 rows and the shapes of split_probs give the same bits on every call.
+  if (dtype == KVHOT_F32 || pl.sp) a.fixed = 1;
   if (!schedule && !pl.grid_ok) pl.mfma = false;
   if (schedule && head_dim <= 128 && is_mixed_list(n_dec)) pl.waves = kMixWaves;
   if (schedule && pl.mfma && n_dec % pl.waves != 0)
