@@ -272,8 +272,10 @@ int kvhot_paged_attention(
  * and decode launches both go to the caller's stream).  Every call on a
  * device shares that device's array, so calls that overlap on one device (on
  * different streams, or from threads without ordering) race; calls ordered
- * on one stream do not.  A call writes every partial it reads, so nothing
- * needs clearing between calls.
+ * on one stream do not.  (Calls that use none of it may overlap: fp32, query
+ * groups that are not a power of two, head_dim 96, and lists without decode
+ * rows.  Their rows are not cut by keys here.)  A call writes every partial it
+ * reads, so nothing needs clearing between calls.
  */
 int kvhot_paged_attention_noalloc(
     const void* q, const int64_t q_strides[3],

@@ -3341,7 +3341,7 @@ extern "C" int64_t kvhot_paged_attention_schedule(
 }
 
 // kvhot_paged_attention's body: validation, then the launches, all on the
-// caller's stream.
+// caller's stream.  whole_rows: a call from the grid cuts no decode row.
 static int paged_attention_impl(
     const void* q, const int64_t q_strides[3], const void* k_cache,
     const int64_t k_cache_strides[4], const void* v_cache,
@@ -3354,8 +3354,8 @@ static int paged_attention_impl(
     int64_t block_size, int64_t num_blocks, float scale, int attn_flags,
     int dtype, int64_t partition_tokens, const int32_t* schedule,
     int64_t num_decode_units, int64_t num_prefill_units, int64_t num_merge_units,
-    int64_t num_prefix_units, int64_t schedule_workspace_bytes, void* workspace, int64_t workspace_bytes,
-    void* stream) {
+    int64_t num_prefix_units, int64_t schedule_workspace_bytes, bool whole_rows, void* workspace,
+    int64_t workspace_bytes, void* stream) {
   clear_error();
   const int64_t es = dtype_size(dtype);
   if (es == 0) return set_error(KVHOT_EINVAL, "paged_attention: bad dtype");
@@ -3460,7 +3460,8 @@ static int paged_attention_impl(
   }
   if (pl.mfma) {
     const int64_t pb = partial_bytes(a.G, head_dim);
-    if (pl.unsplit && !schedule && pl.partials > 0 && (!workspace || workspace_bytes < pl.workspace_bytes(a.G, head_dim))) {
+    if (!schedule && pl.partials > 0 &&
+        (whole_rows || (pl.unsplit && (!workspace || workspace_bytes < pl.workspace_bytes(a.G, head_dim))))) {
       // Without room for partials every row is one partition.
       pl.part_tokens = whole_row_tokens(max_k_len);
       pl.max_parts = 1;
@@ -3550,7 +3551,7 @@ extern "C" int kvhot_paged_attention(
                               q_pos_offsets, num_rows, total_query, max_q_len, max_k_len, num_q_heads,
                               num_kv_heads, head_dim, block_size, num_blocks, scale, attn_flags, dtype,
                               partition_tokens, schedule, num_decode_units, num_prefill_units, num_merge_units,
-                              num_prefix_units, schedule_workspace_bytes, workspace, workspace_bytes, stream);
+                              num_prefix_units, schedule_workspace_bytes, false, workspace, workspace_bytes, stream);
 }
 
 // ------------------------------------------------------------ no-alloc --
@@ -3618,12 +3619,17 @@ extern "C" int kvhot_paged_attention_noalloc(
                                                  num_kv_heads, head_dim, block_size, partition_tokens, dtype);
     if (need < 0) return set_error(static_cast<int>(need), "paged_attention_noalloc: bad sizes");
   }
-  // (unsplit_shape runs from the grid, unsplit, where the partials do not fit.)
-  if (need > KVHOT_NOALLOC_SCRATCH_BYTES && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 &&
-      unsplit_shape(num_q_heads, num_kv_heads, head_dim, block_size, dtype)) {
+  // Shapes of unsplit_shape, and lists without decode rows (whose only partials
+  // are those of prefill units cut by keys), stay off the scratch: they run from
+  // the grid, uncut, so that such calls may overlap on several streams.
+  bool whole_rows = false;
+  if (need > 0 && num_kv_heads > 0 && num_q_heads % num_kv_heads == 0 &&
+      (unsplit_shape(num_q_heads, num_kv_heads, head_dim, block_size, dtype) ||
+       (schedule && num_decode_units == 0 && num_prefix_units == 0))) {
     schedule = nullptr;
     num_decode_units = num_prefill_units = num_merge_units = num_prefix_units = schedule_workspace_bytes = 0;
     need = 0;
+    whole_rows = true;
   }
   if (need > KVHOT_NOALLOC_SCRATCH_BYTES)
     return set_error(KVHOT_EWORKSPACE, "paged_attention_noalloc: the call needs " + std::to_string(need) +
@@ -3639,6 +3645,6 @@ extern "C" int kvhot_paged_attention_noalloc(
                               q_pos_offsets, num_rows, total_query, max_q_len, max_k_len, num_q_heads,
                               num_kv_heads, head_dim, block_size, num_blocks, scale, attn_flags, dtype,
                               partition_tokens, schedule, num_decode_units, num_prefill_units, num_merge_units,
-                              num_prefix_units, schedule_workspace_bytes, ws, need > 0 ? int64_t{KVHOT_NOALLOC_SCRATCH_BYTES} : 0,
+                              num_prefix_units, schedule_workspace_bytes, whole_rows, ws, need > 0 ? int64_t{KVHOT_NOALLOC_SCRATCH_BYTES} : 0,
                               stream);
 }
