@@ -3452,10 +3452,15 @@ static int paged_attention_impl(
                              a.v_sb, a.v_st, a.v_sh, a.o_st, a.o_sh};
     bool aligned = (ptr_or % 16) == 0;
     for (int64_t x : str) aligned = aligned && (x % al) == 0;
-    // Buffer descriptors cover one block: its stride (and the token stride
-    // inside it) must fit their 32-bit ranges.
-    const bool fits = a.k_sb > 0 && a.v_sb > 0 && es * a.k_sb < (1LL << 31) && es * a.v_sb < (1LL << 31) &&
-                      a.k_st > 0 && a.v_st > 0 && 16 * es * a.k_st < (1LL << 31) && 16 * es * a.v_st < (1LL << 31);
+    // Buffer descriptors cover one block, from a kv head's first row to the
+    // block stride: the head's rows must lie within it (blocks whose tokens are
+    // further apart than the blocks themselves run on the VALU kernel), and it
+    // must fit their 32-bit ranges.
+    const auto in_block = [&](int64_t sb, int64_t st) {
+      return st > 0 && sb > 0 && es * sb < (1LL << 31) && 16 * es * st < (1LL << 31) &&
+             (block_size - 1) * st + head_dim <= sb;
+    };
+    const bool fits = in_block(a.k_sb, a.k_st) && in_block(a.v_sb, a.v_st);
     if (!aligned || !fits) pl.mfma = false;
   }
   if (pl.mfma) {
