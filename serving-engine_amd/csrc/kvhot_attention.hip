@@ -211,6 +211,20 @@ __device__ inline int decode_visible_keys(const AttnArgs& a, int row) {
                               static_cast<int64_t>(a.max_parts) * a.part_tokens));
 }
 
+// Bit n: a lane (n, g) with `valid` holds a NaN among o (uniform).  (IEEE
+// maximum, which a NaN passes through: half an instruction per value.)
+template <int N>
+__device__ inline uint32_t nan_row_mask(const f32x4 (&o)[N], bool valid) {
+  float m = 0.f;
+#pragma unroll
+  for (int e = 0; e < N; ++e) {
+    m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, o[e][0]), o[e][1]);
+    m = __builtin_elementwise_maximum(__builtin_elementwise_maximum(m, o[e][2]), o[e][3]);
+  }
+  const uint64_t b = __builtin_amdgcn_ballot_w64(__builtin_isnan(m) && valid);
+  return static_cast<uint32_t>((b | b >> 16 | b >> 32 | b >> 48) & 0xffffu);
+}
+
 // Prefill tiles move their softmax reference only when a score exceeds it by
 // more than this many log2 units, so P <= 2^15: finite as an fp16 operand
 // (largest 65504), and with up to 2^31 keys and |V| < 2^70 the fp32 sums stay
@@ -604,6 +618,9 @@ struct WaveAttn {
       }
   }
 
+  // Bit n: m-row 16 s + n is valid and holds a NaN in O (uniform).
+  __device__ uint32_t nan_rows(int s) const { return nan_row_mask<EPL>(o[s], mval[s]); }
+
   // Row sums over the four lane groups that share an m-row.
   __device__ void row_sums(float (&ltot)[NM]) const {
 #pragma unroll
@@ -804,6 +821,7 @@ struct WaveAttn<F32, D, NM, false> {
     }
   }
   __device__ void store_slot(float* dst, float inv) const { store_row(dst, 0, inv); }
+  __device__ uint32_t nan_rows(int s) const { return nan_row_mask<EPL>(o[s], mval[s]); }
 
   __device__ void row_sums(float (&ltot)[NM]) const {
 #pragma unroll
@@ -813,6 +831,81 @@ struct WaveAttn<F32, D, NM, false> {
     }
   }
 };
+
+// ------------------------------------------------------------ NaN rows --
+// A product of two matrices adds 0 * V where a query does not see a key, and
+// with split probabilities the two parts' products of a V that is infinite:
+// inf + 0 * inf, or inf - inf.  An m-row whose O came out NaN is attended again
+// by attend_row, key by key in fp32 over the keys it sees, and is then what
+// its values say: infinite, NaN, or finite where the offending V is not
+// visible.  (16-bit shapes without split probabilities keep their products.)
+
+// A prefill kernel's AttnArgs, read again from its kernel arguments (it is the
+// only one) rather than held in scalar registers up to a path hardly ever
+// taken: held, they spilled, and calls of 24 to 37 us took 2 to 8% longer than
+// without that path, where they take 1 to 3% longer now.
+typedef const __attribute__((address_space(4))) AttnArgs* late_args_t;
+__device__ inline late_args_t late_args() {
+  late_args_t p = (late_args_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return p;
+}
+
+// Softmax state of one query head: O in lanes (head_dim lane + 64 i).
+template <int D>
+struct RowState {
+  float m = -INFINITY, l = 0.f;
+  float o[(D + 63) / 64] = {};
+  __device__ float inv() const { return l > 0.f ? 1.f / l : 0.f; }
+  __device__ float lse2() const { return l > 0.f ? m + log2f(l) : -INFINITY; }
+};
+
+// One wave: query token t, query head h over keys [k0, k1) of `row`.  Args: a
+// pointer to the kernel's AttnArgs.
+template <class TT, int D, class Args>
+__device__ __attribute__((always_inline)) inline RowState<D> attend_row(Args a, int lane, int row, int64_t t, int h,
+                                                                        int k0, int k1) {
+  using st = typename TT::storage;
+  const int bs = a->bs, kvh = h / a->G;
+  const int32_t* btrow = a->bt + static_cast<int64_t>(row) * a->bt_stride;
+  const int kend = static_cast<int>(min(static_cast<int64_t>(k1), a->bt_stride * bs));
+  const st* qp = static_cast<const st*>(a->q) + t * a->q_st + static_cast<int64_t>(h) * a->q_sh;
+  auto key = [&](const void* p, int64_t sb, int64_t stt, int64_t sh, int tok) {
+    const int64_t id = min(max(static_cast<int64_t>(btrow[tok / bs]), int64_t{0}), a->num_blocks - 1);
+    return static_cast<const st*>(p) + kvh * sh + id * sb + (tok % bs) * stt;
+  };
+  RowState<D> s;
+#pragma nounroll
+  for (int ts = k0; ts < kend; ts += kWave) {
+    const bool valid = ts + lane < kend;
+    float x = -INFINITY;
+    if (valid) {
+      const st* kp = key(a->k, a->k_sb, a->k_st, a->k_sh, ts + lane);
+      float dot = 0.f;
+#pragma nounroll
+      for (int d = 0; d < D; ++d) dot = fmaf(TT::to_float(qp[d]), TT::to_float(kp[d]), dot);
+      x = dot * a->scale_log2;
+    }
+    const float mnew = fmaxf(s.m, wave_max(x));
+    const float muse = mnew == -INFINITY ? 0.f : mnew;
+    const float corr = exp2f(s.m - muse);
+    const float p = valid ? exp2f(x - muse) : 0.f;
+    s.l = s.l * corr + wave_sum(p);
+    s.m = mnew;
+#pragma unroll
+    for (int i = 0; i < (D + 63) / 64; ++i) s.o[i] *= corr;
+    const int n = min(kWave, kend - ts);
+#pragma nounroll
+    for (int j = 0; j < n; ++j) {
+      const float pj = __shfl(p, j, kWave);
+      const st* vp = key(a->v, a->v_sb, a->v_st, a->v_sh, ts + j);
+#pragma unroll
+      for (int i = 0; i < (D + 63) / 64; ++i)
+        if (lane + 64 * i < D) s.o[i] = fmaf(pj, TT::to_float(vp[lane + 64 * i]), s.o[i]);
+    }
+  }
+  return s;
+}
 
 // --------------------------------------------------------------- decode --
 // A decode row's keys are cut into (row, kv head, partition) segments, and a
@@ -896,7 +989,8 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   const int PT = a.part_tokens;
   const int S = a.dec_slots;
   const int P = MR ? a.dec_ranges : W;  // ranges: wave w starts on range w (w < W <= P)
-  const bool fixed = a.fixed != 0;
+  // fp32 rows and split probabilities: the same bits on every call.
+  const bool fixed = SP || std::is_same<TT, F32>::value || a.fixed != 0;
 
   // ---- this wave's range: slices [s0, s1) of part `part` of (row, kvh) ----
   int row = -1, kvh = 0, s0 = 0, s1 = 0, part = 0, nparts = 0, kend = 0;
@@ -1090,10 +1184,24 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
   auto flush = [&]() {
     float lt[1];
     wa.row_sums(lt);
+    uint32_t again = 0;  // m-rows to attend again
+    if constexpr (SP) again = wa.nan_rows(0);
     if (wa.mval[0]) {
       const float inv = lt[0] > 0.f ? 1.f / lt[0] : 0.f;
       wa.store_slot(so + (static_cast<int64_t>(slot) * G + wa.n) * D, inv);
       if (wa.g == 0) sl[slot * G + wa.n] = lt[0] > 0.f ? wa.m[0] + TT::log2(lt[0]) : -INFINITY;
+    }
+    if constexpr (SP) {
+      // (After the stores above, so that the wave's state is not held through
+      // it.  These shapes' waves walk their own range and no other.)
+      for (uint32_t b = again; b; b &= b - 1) {
+        const int hh = __builtin_ctz(b);
+        const RowState<D> rs = attend_row<TT, D>(&a, lane, row, qs, kvh * G + hh, kb, ke);
+#pragma unroll
+        for (int c = 0; c < (D + 63) / 64; ++c)
+          if (lane + 64 * c < D) so[(static_cast<int64_t>(slot) * G + hh) * D + lane + 64 * c] = rs.o[c] * rs.inv();
+        if (lane == 0) sl[slot * G + hh] = rs.lse2();
+      }
     }
     if (lane == 0) {
       skey[4 * slot + 0] = krow;
@@ -2082,15 +2190,41 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
   asm volatile("" : "+v"(el));
   wa.n = el & 15;
   wa.g = el >> 4;
+  uint64_t again = 0;  // m-rows to attend again
+  if constexpr (SP)
+#pragma unroll
+    for (int s = 0; s < NM; ++s) again |= static_cast<uint64_t>(wa.nan_rows(s)) << (16 * s);
 #pragma unroll
   for (int s = 0; s < NM; ++s) {
-    if (!wa.mval[s]) continue;
+    if (!wa.mval[s] || (SP && again >> (16 * s + wa.n) & 1)) continue;
     if (partial)  // (q0 counts from the row's first query, partials from the unit's)
       wa.store_partial_blocks(a, s,
                               static_cast<int64_t>(pbase) + static_cast<int64_t>(q0 - q0g + wa.row_query(a, s)) * pstride,
                               wa.row_head(a, s) - kvh * a.G, ltot[s]);
     else
       wa.store_final_blocks(a, s, qs + q0 + wa.row_query(a, s), ltot[s]);
+  }
+  if constexpr (SP) {
+    for (uint64_t b = again; b; b &= b - 1) {
+      const late_args_t la = late_args();
+      const int i = __builtin_ctzll(b), qi = q0 + i / la->G, hh = i % la->G;
+      const RowState<D> rs =
+          attend_row<TT, D>(la, lane, row, qs + qi, kvh * la->G + hh, k0, causal ? min(klen, off + qi + 1) : klen);
+      const int64_t pi = static_cast<int64_t>(pbase) + static_cast<int64_t>(qi - q0g) * pstride;
+      typename TT::storage* op = static_cast<typename TT::storage*>(la->o) + (qs + qi) * la->o_st +
+                                 static_cast<int64_t>(kvh * la->G + hh) * la->o_sh;
+#pragma unroll
+      for (int c = 0; c < (D + 63) / 64; ++c) {
+        const int d = lane + 64 * c;
+        if (d >= D) continue;
+        if (partial) la->ws_o[(pi * la->G + hh) * D + d] = rs.o[c] * rs.inv();
+        else op[d] = TT::from_float(rs.o[c] * rs.inv());
+      }
+      if (lane == 0) {
+        if (partial) la->ws_lse[pi * la->G + hh] = rs.lse2();
+        else if (la->lse) la->lse[(qs + qi) * la->l_st + static_cast<int64_t>(kvh * la->G + hh) * la->l_sh] = rs.lse2() * kLn2;
+      }
+    }
   }
 }
 
@@ -2225,19 +2359,26 @@ attn_prefill_f32_kernel(const AttnArgs a) {
 #pragma unroll
   for (int s = 0; s < NM; ++s) {
     wa.store_row(so[wave][16 * s + wa.n], s, 1.f);
+    // (A NaN in O is told by the row's maximum.)
+    const bool again = wa.nan_rows(s) >> wa.n & 1;
     if (wa.g == 0) {
-      sm[wave][16 * s + wa.n] = wa.m[s];
+      sm[wave][16 * s + wa.n] = again ? __builtin_nanf("") : wa.m[s];
       sl[wave][16 * s + wa.n] = lt[s];
     }
   }
   __syncthreads();
+  auto row_max = [&](int r) {  // NaN: the row is attended again
+    float mx = sm[0][r];
+#pragma unroll
+    for (int w = 1; w < kPre32Waves; ++w) mx = __builtin_elementwise_maximum(mx, sm[w][r]);
+    return mx;
+  };
   for (int it = threadIdx.x; it < nq * a.G * (D / 4); it += 64 * kPre32Waves) {
     const int r = it / (D / 4), d0 = 4 * (it % (D / 4));
     const int64_t t = qs + q0 + r / a.G;
     if (t >= a.total_q) break;  // (t does not fall as it grows)
-    float mx = sm[0][r];
-#pragma unroll
-    for (int w = 1; w < kPre32Waves; ++w) mx = fmaxf(mx, sm[w][r]);
+    const float mx = row_max(r);
+    if (__builtin_isnan(mx)) continue;
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
     float lsum = 0.f;
     if (mx != -INFINITY) {
@@ -2253,6 +2394,21 @@ attn_prefill_f32_kernel(const AttnArgs a) {
     F32::store4(static_cast<float*>(a.o) + t * a.o_st + static_cast<int64_t>(h) * a.o_sh + d0, acc * inv);
     if (a.lse && d0 == 0)
       a.lse[t * a.l_st + static_cast<int64_t>(h) * a.l_sh] = lsum > 0.f ? (mx + F32::log2(lsum)) * kLn2 : -INFINITY;
+  }
+  // (One look at all rows: lane r's.)
+  const bool bad = lane < nq * a.G && __builtin_isnan(row_max(min(lane, R - 1)));
+  for (uint64_t rows = __builtin_amdgcn_ballot_w64(bad); rows; rows &= rows - 1) {
+    const int r = __builtin_ctzll(rows);
+    const int64_t t = qs + q0 + r / a.G;
+    if (r % kPre32Waves != wave || t >= a.total_q) continue;
+    const late_args_t la = late_args();
+    const int h = kvh * a.G + r % a.G;
+    const RowState<D> rs = attend_row<F32, D>(la, lane, row, t, h, 0, a.causal ? min(klen, off + q0 + r / a.G + 1) : klen);
+#pragma unroll
+    for (int c = 0; c < (D + 63) / 64; ++c)
+      if (lane + 64 * c < D)
+        static_cast<float*>(la->o)[t * la->o_st + static_cast<int64_t>(h) * la->o_sh + lane + 64 * c] = rs.o[c] * rs.inv();
+    if (la->lse && lane == 0) la->lse[t * la->l_st + static_cast<int64_t>(h) * la->l_sh] = rs.lse2() * kLn2;
   }
 }
 
@@ -3437,8 +3593,6 @@ static int paged_attention_impl(
     a.sched = a.merge_units = nullptr;
     n_dec = n_pre = n_mrg = n_pfx = 0;
   }
-  // fp32 rows and the shapes of split_probs give the same bits on every call.
-  if (dtype == KVHOT_F32 || pl.sp) a.fixed = 1;
   if (!schedule && !pl.grid_ok) pl.mfma = false;
   if (schedule && head_dim <= 128 && is_mixed_list(n_dec)) pl.waves = kMixWaves;
   if (schedule && pl.mfma && n_dec % pl.waves != 0)
