@@ -1191,7 +1191,7 @@ __device__ __attribute__((always_inline)) inline void decode_wg(const AttnArgs& 
       wa.store_slot(so + (static_cast<int64_t>(slot) * G + wa.n) * D, inv);
       if (wa.g == 0) sl[slot * G + wa.n] = lt[0] > 0.f ? wa.m[0] + TT::log2(lt[0]) : -INFINITY;
     }
-    if constexpr (SP) {
+    if (SP && __builtin_expect(again != 0, 0)) {
       // (After the stores above, so that the wave's state is not held through
       // it.  These shapes' waves walk their own range and no other.)
       for (uint32_t b = again; b; b &= b - 1) {
@@ -2204,7 +2204,7 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
     else
       wa.store_final_blocks(a, s, qs + q0 + wa.row_query(a, s), ltot[s]);
   }
-  if constexpr (SP) {
+  if (SP && __builtin_expect(again != 0, 0)) {
     for (uint64_t b = again; b; b &= b - 1) {
       const late_args_t la = late_args();
       const int i = __builtin_ctzll(b), qi = q0 + i / la->G, hh = i % la->G;
