@@ -2840,7 +2840,8 @@ static std::vector<PrefixGroup> find_prefix_groups(const int32_t* q_starts, cons
 static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int32_t* q_offs,
                         const int32_t* q_starts, const int32_t* bt, int64_t bt_stride, int64_t bs,
                         int64_t rows, int64_t Hkv, bool causal, int W, int ranges, int64_t groups,
-                        int64_t given_pt, int64_t slice_bytes, int64_t prefix_queries, std::vector<int4>& dec,
+                        int64_t given_pt, int64_t slice_bytes, int64_t prefix_queries, int64_t prefix_units,
+                        std::vector<int4>& dec,
                         std::vector<int4>& mrg, std::vector<int4>& pfx, int64_t& partials) {
   dec.clear();
   mrg.clear();
@@ -2860,13 +2861,11 @@ static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int3
   std::vector<int64_t> pfx_sl(rows, 0), pfx_splits(rows, 0);
   for (const PrefixGroup& pg : pgroups) {
     const int64_t qblocks = (pg.nrows + prefix_queries - 1) / prefix_queries;
-    // Key splits for a device-fill of prefix work-groups (a CU holds two
-    // 4-wave prefill work-groups where it holds one decode work-group): on
-    // 256 rows sharing 1024 keys (D=128, G=4), 512 units (8 splits) took
-    // 74.7 us per call against 76.2 with 256 and 78.2 with 128 (one box):
-    // shorter units outweigh the more fp32 partials to write and fold.
-    const int64_t units = std::max<int64_t>(2 * groups, 1);
-    const int64_t want = (units + qblocks * Hkv - 1) / (qblocks * Hkv);
+    // Key splits for a device-fill of prefix work-groups (prefix_units: on 256
+    // rows sharing 1024 keys, D=128, G=4, 512 units (8 splits) took 74.7 us per
+    // call against 76.2 with 256 and 78.2 with 128, one box: shorter units
+    // outweigh the more fp32 partials to write and fold.)
+    const int64_t want = (prefix_units + qblocks * Hkv - 1) / (qblocks * Hkv);
     const int64_t ks = std::max<int64_t>(1, std::min<int64_t>(want, pg.keys / kMinSplitKeys));
     for (int64_t r = pg.r0; r < pg.r0 + pg.nrows; ++r) {
       pfx_sl[r] = pg.keys / 16;
@@ -3442,20 +3441,25 @@ extern "C" int64_t kvhot_paged_attention_schedule(
     const bool mixed = mixed_launch(head_dim, partition_tokens > 0, has_decode, !pre.empty());
     const int waves = mixed ? kMixWaves : pl.waves;
     const int64_t slice_bytes = 32 * head_dim * dtype_size(dtype);
-    int64_t groups = 0;
+    // 8-wave decode work-groups the device holds at once; shared-prefix units,
+    // which run in a launch of their own, are planned for twice as many (a CU
+    // holds two 4-wave prefill work-groups where it holds one of these)
+    // whichever launch the decode rows are in.  (Planned for twice a mixed
+    // launch's 4-wave groups, 64 rows behind 16384 shared keys beside 64 queries
+    // had 928 units in the place of 512.)
+    int64_t groups = resident_decode_waves(dtype, head_dim, pl.waves, G) / pl.waves;
+    const int64_t prefix_units = std::max<int64_t>(2 * groups, 1);
     if (mixed) {
       int64_t tiles = 0;
       for (size_t i = 0; i < pre.size(); i += 2) tiles += pre[i].w;
       groups = mixed_decode_groups(head_dim, G, cus, static_cast<int64_t>(pre.size() / 2), tiles,
                                    keys * num_kv_heads * slice_bytes / 16);
-    } else {
-      groups = resident_decode_waves(dtype, head_dim, pl.waves, G) / pl.waves;
     }
     const int64_t prefix_queries = prefill_queries(head_dim, G);  // per prefill work-group
     const int ranges = decode_ranges(waves, G, head_dim, partition_tokens > 0);
     if (plan_decode(q_lens, k_lens, q_pos_offsets, q_starts, block_table, bt_row_stride, block_size,
                     num_rows, num_kv_heads, is_causal, waves, ranges, groups, partition_tokens,
-                    slice_bytes, prefix_queries, dec, mrg, pfx, partials)) {
+                    slice_bytes, prefix_queries, prefix_units, dec, mrg, pfx, partials)) {
       if (mixed && !is_mixed_list(static_cast<int64_t>(dec.size() / 2)))
         for (int e = 0; e < kMixWaves; ++e) {  // an empty work-group
           dec.push_back(int4{-1, 0, 0, 0});
