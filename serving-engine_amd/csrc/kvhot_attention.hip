@@ -2979,30 +2979,40 @@ static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int3
     }
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return n[x] > n[y]; });
     const int64_t ng = std::max<int64_t>(std::max<int64_t>(groups, 1), (nseg + W - 1) / W);
-    // (slices, work-group) of the open work-groups, in order; one leaves when
-    // full.  (Looking at the first kMixCandidates in place: popping them off a
-    // heap and pushing all but one back took most of the planner's 1 ms for
-    // 256 rows.)
-    std::set<std::pair<int64_t, int64_t>> open;
-    for (int64_t g2 = 0; g2 < ng; ++g2) open.emplace_hint(open.end(), 0, g2);
-    std::vector<std::vector<Piece>> lpt(ng);
-    std::vector<int> held(static_cast<size_t>(ng * Hkv), 0);  // segments of each kv head per work-group
+    std::vector<std::vector<Piece>> lpt;
     int64_t lmax = 0;
-    for (int sg : order) {
-      const int h = seg_kvh[sg];
-      auto best = open.begin();
-      const int64_t most = best->first + kMixSlack;
-      int seen = 1;
-      for (auto it = std::next(best); it != open.end() && seen < kMixCandidates && it->first <= most; ++it, ++seen)
-        if (held[it->second * Hkv + h] < held[best->second * Hkv + h]) best = it;
-      auto node = open.extract(best);
-      auto& [ld, g2] = node.value();
+    auto whole = [&](int sg) {
       const int64_t s0 = pfx_sl[seg_row[sg]];
-      lpt[g2].push_back(Piece{seg_row[sg], seg_kvh[sg], static_cast<int>(s0), static_cast<int>(s0 + n[sg]), 0, sg});
-      ++held[g2 * Hkv + h];
-      ld += n[sg];
-      lmax = std::max(lmax, ld);
-      if (static_cast<int>(lpt[g2].size()) < W) open.insert(std::move(node));
+      return Piece{seg_row[sg], seg_kvh[sg], static_cast<int>(s0), static_cast<int>(s0 + n[sg]), 0, sg};
+    };
+    // No more segments than work-groups, none empty: each has one to itself.
+    const bool alone = nseg <= ng && n[order.back()] > 0;
+    if (alone) {
+      lmax = n[order[0]];
+    } else {
+      // (slices, work-group) of the open work-groups, in order; one leaves when
+      // full.  (Looking at the first kMixCandidates in place: popping them off a
+      // heap and pushing all but one back took most of the planner's 1 ms for
+      // 256 rows.)
+      std::set<std::pair<int64_t, int64_t>> open;
+      for (int64_t g2 = 0; g2 < ng; ++g2) open.emplace_hint(open.end(), 0, g2);
+      lpt.resize(ng);
+      std::vector<int> held(static_cast<size_t>(ng * Hkv), 0);  // segments of each kv head per work-group
+      for (int sg : order) {
+        const int h = seg_kvh[sg];
+        auto best = open.begin();
+        const int64_t most = best->first + kMixSlack;
+        int seen = 1;
+        for (auto it = std::next(best); it != open.end() && seen < kMixCandidates && it->first <= most; ++it, ++seen)
+          if (held[it->second * Hkv + h] < held[best->second * Hkv + h]) best = it;
+        auto node = open.extract(best);
+        auto& [ld, g2] = node.value();
+        lpt[g2].push_back(whole(sg));
+        ++held[g2 * Hkv + h];
+        ld += n[sg];
+        lmax = std::max(lmax, ld);
+        if (static_cast<int>(lpt[g2].size()) < W) open.insert(std::move(node));
+      }
     }
     const double slice_us = static_cast<double>(slice_bytes) * ng / (kDecodeRateGBs * 1e3);
     // Slices until the cut plan ends, its work-groups taken in order by
@@ -3023,6 +3033,8 @@ static bool plan_decode(const int32_t* q_lens, const int32_t* k_lens, const int3
     }
     if (!any_cut || static_cast<double>(lmax - cut_span) * slice_us <= kMergeLaunchUs) {
       wgs.clear();
+      if (alone)
+        for (int sg : order) wgs.push_back({whole(sg)});
       for (auto& g2 : lpt)
         if (!g2.empty()) wgs.push_back(std::move(g2));
       std::fill(seg_parts.begin(), seg_parts.end(), 1);
@@ -3242,10 +3254,27 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
       partials += nq * ks;
     }
   }
-  std::stable_sort(units.begin(), units.end(), [](const Unit& x, const Unit& y) { return x.tiles > y.tiles; });
-  for (const Unit& un : units) {
-    pre.push_back(un.u);
-    pre.push_back(un.u1);
+  // Longest first, else as they are: a counting sort by tiles (where there are
+  // not many more tile counts than units; an 8192-token prompt's 2048 units took
+  // most of the planner's 62 us by std::stable_sort).
+  pre.reserve(2 * units.size());
+  if (longest <= 4096 + 4 * static_cast<int64_t>(units.size())) {
+    std::vector<int> at(static_cast<size_t>(longest) + 1, 0);  // units of more tiles
+    for (const Unit& un : units)
+      if (un.tiles > 0) ++at[un.tiles - 1];
+    for (int64_t t = longest - 1; t >= 0; --t) at[t] += at[t + 1];
+    pre.resize(2 * units.size());
+    for (const Unit& un : units) {
+      const size_t i = 2 * static_cast<size_t>(at[un.tiles]++);
+      pre[i] = un.u;
+      pre[i + 1] = un.u1;
+    }
+  } else {
+    std::stable_sort(units.begin(), units.end(), [](const Unit& x, const Unit& y) { return x.tiles > y.tiles; });
+    for (const Unit& un : units) {
+      pre.push_back(un.u);
+      pre.push_back(un.u1);
+    }
   }
 }
 
