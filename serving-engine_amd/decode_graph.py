@@ -19,14 +19,12 @@ whose counts differ from the recorded ones records the graph again.
 """
 from __future__ import annotations
 
-import ctypes
-
 import numpy as np
 import torch
 
 from . import _lib
 from .block import BLOCK_SIZE
-from .paged_attention_kernel import build_slot_mapping, schedule_key
+from .paged_attention_kernel import build_slot_mapping, pinned_units, plan_units, schedule_key
 
 
 class DecodeStepGraph:
@@ -108,21 +106,11 @@ class DecodeStepGraph:
         """Launch list of the step's attention calls from the host arrays."""
         r, mb = self.r, self.max_blocks
         hq, hkv, d, bs, pt, causal, dt = self.shape
-        lib = _lib.load()
-        cnt = [ctypes.c_int64(0) for _ in range(5)]  # decode, prefill, merge, workspace, prefix
-        outs = tuple(ctypes.byref(c) for c in cnt)
         base = a.ctypes.data  # q_lens, k_lens, q_starts, q_pos_offsets, block table: int32 views of `a`
         args = (base, base + 4 * r, base + 8 * r, base + 12 * r, base + 16 * r, mb, r, hq, hkv, d, bs, pt,
                 1 if causal else 0, dt)
-        total = lib.kvhot_paged_attention_schedule(*args, None, 0, *outs)
-        if total < 0:
-            _lib.check(int(total), "kvhot_paged_attention_schedule")
-        units = torch.empty((max(int(total), 1), 8), dtype=torch.int32, pin_memory=True)
-        if total > 0:
-            got = lib.kvhot_paged_attention_schedule(*args, units.data_ptr(), total, *outs)
-            if got != total:
-                _lib.check(-1 if got >= 0 else int(got), "kvhot_paged_attention_schedule")
-        return units, tuple(int(c.value) for c in cnt)
+        units, counts = plan_units(args, r, int(a[r:2 * r].max()), hkv)
+        return pinned_units(units), counts
 
     # -- the recorded step -------------------------------------------------
 

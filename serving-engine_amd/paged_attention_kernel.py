@@ -67,6 +67,35 @@ def schedule_key(device, hq, hkv, d, bs, pt, causal, dtype):
     return (hq, hkv, d, bs, pt, bool(causal), dtype, str(device))
 
 
+def plan_units(args, rows, max_k, hkv):
+    """(units [n, 8] int32, (n_decode, n_prefill, n_merge, workspace bytes,
+    n_prefix)) of kvhot_paged_attention_schedule for the arguments `args`
+    before its outputs: one run of the planner, into a list of as many units
+    as the step has 16-token slices at most (up to LIST_UNITS); a longer list
+    takes a second."""
+    lib = _lib.load()
+    counts = [ctypes.c_int64(0) for _ in range(5)]
+    outs = tuple(ctypes.byref(c) for c in counts)
+    room = min(LIST_UNITS, 256 + (max_k // BLOCK_SIZE + 1) * rows * hkv)
+    units = np.empty((room, 8), dtype=np.int32)
+    total = int(lib.kvhot_paged_attention_schedule(*args, units.ctypes.data, room, *outs))
+    if total > room:
+        units = np.empty((total, 8), dtype=np.int32)
+        if lib.kvhot_paged_attention_schedule(*args, units.ctypes.data, total, *outs) != total:
+            total = -1
+    if total < 0:
+        _lib.check(total, "kvhot_paged_attention_schedule")
+    return units[:total], tuple(int(c.value) for c in counts)
+
+
+def pinned_units(units):
+    """A pinned copy of a plan's units (one unit at least, for a stable copy
+    source)."""
+    staged = torch.empty((max(len(units), 1), 8), dtype=torch.int32, pin_memory=True)
+    staged.numpy()[:len(units)] = units
+    return staged
+
+
 def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
     """(device units, n_decode, n_prefill, n_merge, workspace bytes, n_prefix)
     of kvhot_paged_attention_schedule for this step, built once per attention
@@ -83,30 +112,14 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
     host_off = metadata["host_q_pos_offsets"]
     host_qs = metadata["host_q_starts"]
     host_bt = metadata["host_block_table"]
-    lib = _lib.load()
-    # decode, prefill, merge units; workspace bytes; shared-prefix units
-    counts = [ctypes.c_int64(0) for _ in range(5)]
     args = (host_q.ctypes.data, host_k.ctypes.data, host_qs.ctypes.data, host_off.ctypes.data,
             host_bt.ctypes.data if host_bt.size else None, host_bt.shape[1] if host_bt.ndim == 2 else 0,
             len(host_q), hq, hkv, d, bs, pt, 1 if causal else 0, dtype)
-    outs = tuple(ctypes.byref(c) for c in counts)
-    # One call of the planner fills a list of as many units as the step has
-    # 16-token slices at most (up to LIST_UNITS); a longer one takes a second.
-    room = min(LIST_UNITS, 256 + (_host_max(metadata, "max_k_len", "k_lens") // BLOCK_SIZE + 1) * len(host_q) * hkv)
-    units = np.empty((room, 8), dtype=np.int32)
-    total = int(lib.kvhot_paged_attention_schedule(*args, units.ctypes.data, room, *outs))
-    if total > room:
-        units = np.empty((total, 8), dtype=np.int32)
-        if lib.kvhot_paged_attention_schedule(*args, units.ctypes.data, total, *outs) != total:
-            total = -1
-    if total < 0:
-        _lib.check(total, "kvhot_paged_attention_schedule")
-    if total == 0:
+    units, counts = plan_units(args, len(host_q), _host_max(metadata, "max_k_len", "k_lens"), hkv)
+    if len(units) == 0:
         hit = None
     else:
-        staged = torch.empty((total, 8), dtype=torch.int32, pin_memory=True)
-        staged.numpy()[:] = units[:total]
-        hit = (staged.to(device, non_blocking=True),) + tuple(int(c.value) for c in counts)
+        hit = (pinned_units(units).to(device, non_blocking=True),) + counts
     cache[key] = hit
     return hit
 
