@@ -4,9 +4,11 @@
 //
 // Every function here answers the ordinary call only, after checking all that
 // the Python function of the same name checks, and returns None before it has
-// done anything when a check fails or when something it needs (a launch list,
-// a workspace) is not there yet; the Python function then takes the call, does
-// that preparation or raises.  Nothing is kept between calls: pointers, shapes
+// done anything when a check fails, when something it needs (a launch list,
+// a workspace) is not there yet or when the library refuses the launch; the
+// Python function then takes the call, does that preparation or raises.  (Where
+// layer()'s attention is refused its append is queued already, and its answer
+// says so.)  Nothing is kept between calls: pointers, shapes
 // and strides are read from the tensors each time.
 //
 // Measured, Python with ctypes before -> here, calls queued back to back on one
@@ -209,13 +211,14 @@ PyObject* or_none(F f) {
   return r;
 }
 
+// f() without the GIL, which is taken again whichever way f ends.
 template <class F>
 int without_gil(F f) {
-  int status;
-  Py_BEGIN_ALLOW_THREADS
-  status = f();
-  Py_END_ALLOW_THREADS
-  return status;
+  struct Released {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Released() { PyEval_RestoreThread(state); }
+  } released;
+  return f();
 }
 
 Tensor lse_of(const Tensor& q) {
@@ -267,7 +270,8 @@ PyObject* py_append(PyObject*, PyObject* const* a, Py_ssize_t n) {
 }
 
 // layer(kv_cache, heads, dim, key, value, layer, slots, query, metadata, scale, pt, flags, workspaces)
-//   -> o [1, S, Hq, D] | None: the append, then causal attention.
+//   -> o [1, S, Hq, D] | None | False: the append, then causal attention; False
+//   where the append is queued and the library then refused the attention.
 PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
   return or_none([&]() -> PyObject* {
     Append ap;
@@ -291,11 +295,15 @@ PyObject* py_layer(PyObject*, PyObject* const* a, Py_ssize_t n) {
     at_.hkv = ap.heads;
     if (!at_.check(a[8], a[9], pt, true, static_cast<int>(flags), a[12])) return nullptr;
     const Tensor o = at::empty_like(at_.q, at_.q.options().requires_grad(false)), l = lse_of(at_.q);
-    const int status = without_gil([&] {
-      const int rc = ap.launch(at_.stream);
-      return rc != 0 ? rc : at_.launch(o, l);
-    });
-    if (status != 0) return nullptr;
+    if (without_gil([&] { return ap.launch(at_.stream); }) != 0) return nullptr;
+    // (An exception here, from a library call that could not form its message,
+    // is such a refusal too.)
+    int status = -1;
+    try {
+      status = without_gil([&] { return at_.launch(o, l); });
+    } catch (...) {
+    }
+    if (status != 0) Py_RETURN_FALSE;
     return THPVariable_Wrap(o.unsqueeze(0));
   });
 }

@@ -161,14 +161,18 @@ def hip_paged_attention_forward(module, query, key, value, attention_mask, scali
     paged_metadata.  Returns ([1, S, Hq, D], None)."""
     cache: _PagedKVCache = kwargs["cache"]
     if type(cache) is _PagedKVCache:
-        # Both launches from one native call (None: a call for the code below).
+        # Both launches from one native call (None: a call for the code below;
+        # False: the attention is, its append is queued).
         o = _lib.native().layer(
             cache.kv_cache, cache.num_kv_heads, cache.head_dim, key, value, module.layer_idx, kwargs["write_index"],
             query, kwargs["paged_metadata"], scaling, _attention.DEFAULT_PARTITION_TOKENS, _lib.KVHOT_CAUSAL,
             _attention._WORKSPACES)
-        if o is not None:
+        if isinstance(o, torch.Tensor):
             return o, None
-    cache.write(key, value, module.layer_idx, kwargs["write_index"])
+    else:
+        o = None
+    if o is None:
+        cache.write(key, value, module.layer_idx, kwargs["write_index"])
     k_cache_blocks, v_cache_blocks = cache.blocks(module.layer_idx)
     q = query.transpose(1, 2).squeeze(0)  # [S, Hq, D]
     o, _ = paged_flash_attention(

@@ -27,10 +27,11 @@ class _Counted:
     """kvhot_torch, with the calls it took counted."""
 
     def __init__(self, mod):
-        self.mod, self.taken = mod, 0
+        self.mod, self.taken, self.names = mod, 0, []
 
     def __getattr__(self, name):
         def call(*args):
+            self.names.append(name)
             r = getattr(self.mod, name)(*args)
             self.taken += r is not None
             return r
@@ -48,6 +49,65 @@ def test_cpu_calls_are_left_alone():
     assert n.layer(kv, 2, 64, k, k, 0, slots, torch.zeros(1, 4, 2, 64), {}, 0.1, 0, 1, {}) is None
     for f in (n.append, n.attention, n.layer):  # too few arguments, and objects that are no tensors
         assert f() is None and f(*[None] * 13) is None
+
+
+@pytest.mark.parametrize("answer,writes", [(None, 1), (False, 0)])
+def test_a_refused_layer_appends_once(monkeypatch, answer, writes):
+    """layer() answers None before the append and False after it."""
+    runner, lib = sea_module("model_runner"), sea_module("_lib")
+    calls = []
+
+    class _Native:
+        def layer(self, *args):
+            return answer
+
+    def _attention(*args, **kw):
+        calls.append("attention")
+        raise RuntimeError("refused")
+
+    monkeypatch.setattr(lib, "_NATIVE", _Native())
+    monkeypatch.setattr(runner._PagedKVCache, "write", lambda self, *args: calls.append("write"))
+    monkeypatch.setattr(runner, "paged_flash_attention", _attention)
+
+    class _Module:
+        layer_idx = 0
+
+    cache = runner._PagedKVCache(torch.zeros(1, 2, 3, 16, 2, 64))
+    k = torch.zeros(1, 2, 2, 64)
+    with pytest.raises(RuntimeError, match="refused"):
+        runner.hip_paged_attention_forward(_Module(), torch.zeros(1, 4, 2, 64), k, k, None, 0.1, cache=cache,
+                                           write_index=torch.zeros(2, dtype=torch.int64), paged_metadata={})
+    assert calls == ["write"] * writes + ["attention"]
+
+
+@pytest.mark.gpu
+def test_attention_refused_after_the_append(cuda, sea, wl, monkeypatch):  # noqa: F811
+    """A query whose head_dim is not unit-stride, which the library refuses:
+    the step's K/V are appended once, and the refusal is raised."""
+    lib = sea_module("_lib")
+    w = custom(wl, ROWS, 8, 2, 64, torch.bfloat16)
+    T = wl.make_tensors(w, cuda)
+    cache = sea._PagedKVCache(T.kv_cache)
+    meta = wl.metadata_tensors(w, cuda)
+    kc, vc = cache.blocks(0)
+    sea.paged_flash_attention(T.q, kc, vc, meta, 8, 2, 0.125)  # builds the launch list and the workspace
+    native = _Counted(lib.native())
+    monkeypatch.setattr(lib, "_NATIVE", native)
+
+    class _Module:
+        layer_idx = 0
+
+    announce("attention refused after the append (append launch only)")
+    q4 = T.q.transpose(0, 1).unsqueeze(0)
+    bad = torch.stack([q4, q4], -1)[..., 0]
+    assert bad.stride(-1) == 2
+    with pytest.raises(Exception, match="unit-stride"):
+        sea.hip_paged_attention_forward(_Module(), bad, T.new_k, T.new_v, None, 0.125, cache=cache,
+                                        write_index=T.slot_mapping, paged_metadata=meta)
+    torch.cuda.synchronize()
+    assert native.names == ["layer", "attention"]  # (no append of its own)
+    got = T.kv_cache[0].reshape(2, -1, 2, 64)[:, T.slot_mapping.long()]
+    assert torch.equal(got[0], T.new_k[0].transpose(0, 1)) and torch.equal(got[1], T.new_v[0].transpose(0, 1))
 
 
 def _layer(sea, w, T, meta, q4, k4, v4, slots, scale):
