@@ -51,7 +51,9 @@ enum {
 enum {
   KVHOT_CAUSAL = 1,        /* key j is visible to query i iff j <= q_pos_offset + i */
   KVHOT_DETERMINISTIC = 2, /* bitwise-repeatable out and lse: decode waves walk their
-                              planned key ranges in order, with no run-time sharing */
+                              planned key ranges in order, with no run-time sharing
+                              (fp32 calls, query groups that are not a power of two
+                              and head_dim 96 always do) */
   KVHOT_VERIFY_BLOCKS = 4  /* decode waves check the first block of their range that
                               the launch list took from the host copy of the block
                               table against the device table, and use the device
@@ -186,7 +188,9 @@ int64_t kvhot_paged_attention_workspace_bytes(
  * before the decode launch).
  * partition_tokens > 0 (a multiple of 32 up to 2^20) first cuts every decode
  * row into partitions of that many keys, which are then never cut further;
- * 0 leaves the cuts to the planner.  *workspace_bytes receives the workspace
+ * 0 leaves the cuts to the planner.  fp32 calls have no schedule, nor have
+ * query groups that are not a power of two and head_dim 96 with
+ * partition_tokens > 0 (the unit count is 0).  *workspace_bytes receives the workspace
  * the attention call needs with this schedule (0: none).  Returns the total
  * unit count (units are written when `units` is non-NULL and capacity_units
  * suffices) or a negative KVHOT_E* code.  A schedule depends only on the
@@ -226,12 +230,17 @@ int64_t kvhot_paged_attention_schedule(
  * large (a shorter one fails with KVHOT_EWORKSPACE before any launch); or
  * NULL, and then partition_tokens (keys per decode partition; 0 picks a
  * size, otherwise a multiple of 32 up to 2^20) and
- * kvhot_paged_attention_workspace_bytes apply.  Decode waves of one
- * work-group share out their slices at run time (the waves of a CU stream at
- * different rates), so the summation order, and with it the last bits of out
+ * kvhot_paged_attention_workspace_bytes apply (fp32 rows are left whole where
+ * partition_tokens is given).  A workspace that is missing or too small is an
+ * error, except that without a schedule fp32 calls, query groups that are not a
+ * power of two and head_dim 96 then leave their rows whole.  Decode waves of
+ * one work-group share out their slices at run time (the waves of a CU stream
+ * at different rates), so the summation order, and with it the last bits of out
  * and lse, can differ from call to call; with KVHOT_DETERMINISTIC in
  * attn_flags every wave walks its planned range alone and repeated calls
- * give the same bits (the work-group then ends with its slowest wave).
+ * give the same bits (the work-group then ends with its slowest wave).  fp32
+ * calls, query groups that are not a power of two and head_dim 96 run so
+ * without it too.
  * Other attn_flags bits are invalid.  lse may be NULL.  out has the dtype of
  * q, k_cache and v_cache; lse is fp32.  Replaces paged_flash_attention +
  * paged_flash_fwd_kernel (serving_engine/paged_attention_kernel.py:16-160).

@@ -94,7 +94,8 @@ struct AttnArgs {
   int32_t dec_ranges; // range descriptors per decode work-group (its waves, or 4x them)
   // KVHOT_DETERMINISTIC: every decode wave walks exactly its planned range,
   // in order (no claiming from other waves), so each partial sum, and with it
-  // out and lse, is the same bits on every call.
+  // out and lse, is the same bits on every call.  (fp32 rows and the shapes of
+  // split_probs always do.)
   int32_t fixed;
   // KVHOT_VERIFY_BLOCKS: decode waves check a launch list's first block.
   int32_t verify;
@@ -237,7 +238,10 @@ constexpr float kLazyRescale = 15.f;
 // one and what the rounding left (P = hi + lo to 2^-17 in bf16, 2^-22 in
 // fp16), so that an output carries its own rounding only: against fp64, bf16
 // outputs of random inputs are off by 0.0017 in relative L2, as with fp32
-// probabilities, and by 0.0023 with rounded ones.  It costs a second PV
+// probabilities, and by 0.0023 with rounded ones.  (Over decode, prefill and
+// mixed calls of five shapes, bf16 and fp16, the outputs' error is that of the
+// VALU kernel with fp32 probabilities to four digits, the LSE's between 0.96
+// and 1.06 of its 4.5e-8.)  It costs a second PV
 // product (1.5 times the MFMAs) and 5 VALU instructions per pair of
 // probabilities.
 template <class TT, int D, int NM, bool SP = false>
@@ -926,7 +930,12 @@ __device__ __attribute__((always_inline)) inline RowState<D> attend_row(Args a, 
 // After a barrier the first wave of each segment merges that segment's slots.
 // With KVHOT_DETERMINISTIC (AttnArgs::fixed) a wave claims from its own range
 // only and stops when it is used up: slices are summed in the same order on
-// every call.
+// every call.  fp32 rows and split probabilities always run so: they gave the
+// same bits on every call on the VALU kernel.  (It costs nothing where a
+// work-group holds a few segments cut to equal ranges -- 64 rows of 128 to 2048
+// keys, 24 / 8 heads, 49.0 us shared out, 50.0 fixed -- and most where each wave
+// has a whole segment: 200 rows of 100 to 3000 keys 197 against 261, 256 rows of
+// 256 to 2048 187 against 237.)
 // A segment that is one of several partitions of its row stores an (LSE, O)
 // partial to HBM instead, and attn_merge_kernel combines the partitions in a
 // second launch.  (Merging across work-groups inside one launch needs a
@@ -2047,8 +2056,10 @@ __device__ __attribute__((always_inline)) inline void prefill_wg(const AttnArgs&
     }
     // Every wave runs every tile of the unit: a tile wholly past a wave's
     // causal limit is masked like the diagonal one (P = 0), which keeps the
-    // phase one straight block.  Such tiles are at most one per wave, the
-    // waves of a work-group being 16*NM/G queries apart.
+    // phase one straight block.  The waves of a work-group being 16*NM/G queries
+    // apart, the first of PW waves has up to (PW - 1) * 16*NM/G / kPreKeys + 1
+    // such tiles: at most 1 for groups of 4 heads and more, 6 at head_dim 64 and
+    // 3 at head_dim 128 for G = 1.
     auto phase = [&](auto S_, int t) {
       constexpr int S = decltype(S_)::value;
       if (issuer && t + LEAD < ntiles) issue((S + LEAD) & 3, t + LEAD);
@@ -2606,9 +2617,12 @@ static bool mfma_shape_ok(int64_t Hq, int64_t Hkv, int64_t D, int64_t bs, int dt
 // groups that are not a power of two, and head_dim 96.
 static bool split_probs(int64_t G, int64_t D) { return D == 96 || (G & (G - 1)) != 0; }
 
-// Calls launch lists are built for: the 16-bit shapes (fixed partitions of
-// those of split_probs run from the grid, which gives each its own
-// work-group).  Grid -> list for 24 / 8 heads at head_dim 128 (us): 64 rows of
+// Calls launch lists are built for: the 16-bit shapes, those of split_probs
+// without fixed partitions only (the decode kernel that takes several ranges per
+// wave, as a list of fixed partitions has, is not built for them, and one range per
+// wave would be no faster than the grid: 16 rows of 8192 keys, 24 / 8 heads, 180 us
+// from the grid in 512-token partitions, 86 from a list without; 32 / 8 heads 88
+// from a list with them).  Grid -> list for 24 / 8 heads at head_dim 128 (us): 64 rows of
 // 128 to 2048 keys 85 -> 48, 200 rows of 100 to 3000 295 -> 196, 128 rows behind
 // 1024 shared keys 158 -> 50, 56 rows beside eight 512-token prompts 130 -> 76,
 // 64 queries on 16448 keys 519 -> 41, 13 rows beside 5 chunks of up to 300
@@ -2647,8 +2661,9 @@ constexpr int64_t kGridWaves = 256 * 8;
 // Without a schedule, decode rows are cut into partitions of part_tokens keys
 // (0: W * wave_slices slices, so no wave walks more than that many) and the
 // grid enumerates (head group, partition, row).  wave_slices is
-// KVHOT_SLICES_PER_WAVE; for shapes that never have launch lists, fewer (at
-// least 2) when the rows' slices would not fill kGridWaves waves.
+// KVHOT_SLICES_PER_WAVE; for the shapes of unsplit_shape, which no fixed split
+// was promised, fewer (at least 2) when the rows' slices would not fill
+// kGridWaves waves.
 static Plan make_plan(int64_t rows, int64_t max_q, int64_t max_k, int64_t Hq,
                       int64_t Hkv, int64_t D, int64_t bs, int64_t part_tokens,
                       int dtype) {
@@ -3284,8 +3299,13 @@ static void plan_prefill(const int32_t* q_lens, const int32_t* k_lens, const int
 // the slots stays free, since work-groups do not spread evenly enough to take
 // all (247 units and 265 decode work-groups on 512 slots 55.5 us, 254 of them
 // 48.0).  Where the prefill units take more than a round of the slots and as
-// long as the decode rows: all slots' worth of smaller ones, which then fill
-// the end of the launch too.  Measured with 256 / 512 decode work-groups (us):
+// long as the decode rows: all slots' worth of smaller ones.  (Those past a whole
+// turn of attn_mixed_kernel come after the last prefill unit: about half of
+// them, where the plan makes 511 or less.  A plan that packs more than 4 segments
+// to a work-group of these makes more work-groups than this asks for: 256 rows of
+// 8 kv heads are 512, and no longer all start at once.  They still gain by one
+// launch: 256 rows behind 1024 shared keys beside 225 queries 117.6 us as two,
+// 100.2 as one.)  Measured with 256 / 512 decode work-groups (us):
 // 64 decode rows of 128 to 2048 beside 448 queries on 960 keys 59 / 72, 56
 // rows beside eight whole 512-token prompts 76 / 91; 4 rows of 20,000 to 30,000
 // beside two 1024-token chunks on up to 4000 156 / 145, 56 rows beside eight

@@ -161,10 +161,12 @@ def paged_flash_attention(q, k_cache, v_cache, metadata, num_q_heads, num_kv_hea
     build_paged_batch_metadata().  Returns ``o`` shaped and strided like q
     (``torch.empty_like(q)``) and ``l`` = natural-log LSE, fp32
     [total_query, num_q_heads].  Extensions: ``partition_tokens`` cuts
-    decode rows into split-K partitions of at most that many keys;
+    decode rows into split-K partitions of at most that many keys (fp32 rows
+    are then left whole);
     ``deterministic=True`` makes repeated calls on the same inputs give the
     same bits (decode waves then do not share out slices at run time, which
-    costs some speed), as the reference's serial key loop does.
+    costs some speed), as the reference's serial key loop does.  fp32 calls,
+    query groups that are not a power of two and head_dim 96 always do.
     ``verify_block_table=True`` makes decode waves check the first block of
     their range, which the launch list takes from
     ``metadata["host_block_table"]``, against ``metadata["block_table"]``

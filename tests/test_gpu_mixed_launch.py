@@ -1,5 +1,6 @@
 """Prefill units and decode work-groups of one launch, against the fp64 oracle:
-both kinds in turns, fewer than a turn of either, the smallest of both."""
+up to a turn of 256 of either and more, the smallest of both.  (Whole turns at
+every shape: test_gpu_new_plans.py.)"""
 import math
 
 import pytest
@@ -11,7 +12,7 @@ from test_gpu_parity import announce, assert_attention, hip_step, oracle_step, w
 pytestmark = pytest.mark.gpu
 
 SPECS = {
-    # 256 decode work-groups and as many prefill units, and more
+    # about a turn of both kinds where there are 8 kv heads, less or more elsewhere
     "turns": [(1, 90 + 61 * (i % 17), 89 + 61 * (i % 17)) for i in range(40)] + [(300, 400, 100), (513, 513, 0), (270, 300, 30)],
     # slices, ranges and blocks around their edges; a decode row without a key
     "edges": [(1, 1, 0), (1, 16, 15), (2, 2, 0), (1, 17, 16), (0, 5, 5), (1, 129, 128), (33, 65, 32), (1, 1030, 1029),
@@ -36,6 +37,8 @@ def test_mixed_launch(cuda, sea, wl, hq, hkv, d, dtype, spec):  # noqa: F811
     meta = wl.metadata_tensors(w, cuda)
     o, l = hip_step(sea, wl, w, T, meta=meta)
     assert_attention(w, o, l, ref_o, ref_l, rows=rows)
+    (_, n_dec, n_pre, _, _, n_pfx), = meta["_schedules"].values()
+    assert n_dec % 8 == 4 and n_pre > n_pfx  # a list for one launch of both kinds
     kc, vc = sea._PagedKVCache(T.kv_cache).blocks(0)
     scale = 1.0 / math.sqrt(d)
     for kw in (dict(deterministic=True), dict(verify_block_table=True), dict(partition_tokens=64)):

@@ -391,8 +391,9 @@ SHAPES = [
 
 
 def mfma_shape(hq, hkv, d, dtype):
-    """Shapes the MFMA kernels take: bf16/fp16, head_dim 64/128/256, query
-    groups of 1 to 16 heads (powers of two); the rest run the VALU kernel."""
+    """Shapes with launch lists of fixed partitions: bf16/fp16, head_dim
+    64/128/256, query groups of 1 to 16 heads (powers of two).  The rest run
+    from the padded grid."""
     return dtype in (torch.bfloat16, torch.float16) and d in (64, 128, 256) and hq // hkv in (1, 2, 4, 8, 16)
 
 
@@ -406,7 +407,7 @@ def test_shapes_mixed_batch(cuda, sea, wl, hq, hkv, d, dtype):
     o, l = hip_step(sea, wl, w, T, partition_tokens=64, meta=meta)
     live = [i for i, x in enumerate(w.rows) if x.q_len > 0]
     assert_attention(w, o, l, ref_o, ref_l, rows=live)
-    # the path that ran: a launch list (MFMA kernels) exactly for the MFMA shapes
+    # the path that ran: a launch list of 64-key partitions, or the grid
     plans = [p for p in meta.get("_schedules", {}).values() if p is not None]
     assert bool(plans) == mfma_shape(hq, hkv, d, dtype), (hq, hkv, d, dtype)
 
