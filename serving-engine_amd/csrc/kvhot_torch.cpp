@@ -38,7 +38,7 @@ decltype(&kvhot_reshape_and_cache) g_append = nullptr;
 // Keys of the metadata dict and of its launch lists.
 struct Names {
   PyObject *q_lens, *k_lens, *q_starts, *q_pos_offsets, *block_table, *block_table_row_stride, *max_q_len, *max_k_len,
-      *host_q_lens, *schedules;
+      *host_q_lens, *schedules, *schedule_streams;
 } g_names;
 
 // The plain torch.Tensor behind o, with memory on a GPU.  (Subclasses and
@@ -118,6 +118,20 @@ struct Attention {
   int flags;
   void* stream;
 
+  // Whether the stream comes after the copy of the launch list of `key`
+  // (_order_list's record; a list without one is taken as it is).
+  bool list_ordered(PyObject* meta, PyObject* key) const {
+    PyObject* all = PyDict_GetItemWithError(meta, g_names.schedule_streams);
+    PyObject* rec = all && PyDict_CheckExact(all) ? PyDict_GetItemWithError(all, key) : nullptr;
+    if (!rec) return !PyErr_Occurred();
+    if (!PyTuple_CheckExact(rec) || PyTuple_GET_SIZE(rec) != 2 || !PySet_Check(PyTuple_GET_ITEM(rec, 1))) return false;
+    PyObject* h = PyLong_FromLongLong(static_cast<long long>(reinterpret_cast<intptr_t>(stream)));
+    if (!h) return false;
+    const int in = PySet_Contains(PyTuple_GET_ITEM(rec, 1), h);
+    Py_DECREF(h);
+    return in == 1;
+  }
+
   // q, the pool and hkv are set; the rest from the metadata.
   bool check(PyObject* meta, PyObject* scale_o, int64_t pt_, bool causal, int flags_, PyObject* workspaces) {
     if (!PyDict_CheckExact(meta) || !PyDict_CheckExact(workspaces) || !PyFloat_Check(scale_o)) return false;
@@ -126,6 +140,7 @@ struct Attention {
     flags = flags_;
     const c10::Device d = q.device();
     const int64_t hq = q.size(1), dim = q.size(2);
+    stream = c10::hip::getCurrentHIPStream(d.index()).stream();
     const int dt = dtype_code(q);
     if (dt < 0 || hkv <= 0 || hq <= 0 || hq % hkv != 0 || q.size(0) == 0 || dim == 0) return false;
     if (!gpu_tensor(PyDict_GetItemWithError(meta, g_names.q_lens), q_lens) || q_lens.dim() < 1) return false;
@@ -154,8 +169,9 @@ struct Attention {
                                     (long long)pt, causal ? Py_True : Py_False, dt, name);
       if (!key) return false;
       PyObject* hit = PyDict_GetItemWithError(lists, key);
+      const bool ordered = hit && (hit == Py_None || list_ordered(meta, key));
       Py_DECREF(key);
-      if (!hit) return false;
+      if (!ordered) return false;
       if (hit != Py_None) {
         if (!PyTuple_CheckExact(hit) || PyTuple_GET_SIZE(hit) != 6) return false;
         // (device units, decode, prefill, merge units, workspace bytes, prefix units)
@@ -171,7 +187,6 @@ struct Attention {
       need = g_workspace_bytes(rows, q.size(0), max_q, max_k, hq, hkv, dim, block_size, pt, dt);
       if (need < 0) return false;
     }
-    stream = c10::hip::getCurrentHIPStream(d.index()).stream();
     if (need > 0) {  // the stream's workspace, made by the first call that needs it
       PyObject* key = Py_BuildValue("(iL)", static_cast<int>(d.index()),
                                     static_cast<long long>(reinterpret_cast<intptr_t>(stream)));
@@ -341,5 +356,6 @@ PyMODINIT_FUNC PyInit_kvhot_torch(void) {
   g.max_k_len = PyUnicode_InternFromString("max_k_len");
   g.host_q_lens = PyUnicode_InternFromString("host_q_lens");
   g.schedules = PyUnicode_InternFromString("_schedules");
+  g.schedule_streams = PyUnicode_InternFromString("_schedule_streams");
   return PyModule_Create(&kModule);
 }

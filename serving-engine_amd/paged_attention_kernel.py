@@ -67,6 +67,23 @@ def schedule_key(device, hq, hkv, d, bs, pt, causal, dtype):
     return (hq, hkv, d, bs, pt, bool(causal), dtype, str(device))
 
 
+def _order_list(metadata, key, hit, device):
+    """Orders the current stream after the copy of launch list `hit`, which the
+    first call of its shape queued on its own stream.  The streams ordered so
+    far are kept beside the copy's event in metadata["_schedule_streams"]
+    (a list put into the metadata by its maker has no entry, and is taken as it
+    is)."""
+    ordered = metadata.get("_schedule_streams", {}).get(key)
+    if hit is None or ordered is None or torch.cuda.is_current_stream_capturing():
+        return  # (a capture began after the device was waited for)
+    stream = torch.cuda.current_stream(device)
+    event, streams = ordered
+    if stream.cuda_stream not in streams:
+        stream.wait_event(event)
+        hit[0].record_stream(stream)
+        streams.add(stream.cuda_stream)
+
+
 def plan_units(args, rows, max_k, hkv):
     """(units [n, 8] int32, (n_decode, n_prefill, n_merge, workspace bytes,
     n_prefix)) of kvhot_paged_attention_schedule for the arguments `args`
@@ -107,6 +124,7 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
     key = schedule_key(device, hq, hkv, d, bs, pt, causal, dtype)
     cache = metadata.setdefault("_schedules", {})
     if key in cache:
+        _order_list(metadata, key, cache[key], device)
         return cache[key]
     host_k = metadata["host_k_lens"]
     host_off = metadata["host_q_pos_offsets"]
@@ -120,6 +138,10 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
         hit = None
     else:
         hit = (pinned_units(units).to(device, non_blocking=True),) + counts
+        stream = torch.cuda.current_stream(device)
+        event = torch.cuda.Event()
+        event.record(stream)
+        metadata.setdefault("_schedule_streams", {})[key] = (event, {stream.cuda_stream})
     cache[key] = hit
     return hit
 
