@@ -126,6 +126,10 @@ def _schedule(metadata, device, hq, hkv, d, bs, pt, causal, dtype):
     if key in cache:
         _order_list(metadata, key, cache[key], device)
         return cache[key]
+    if torch.cuda.is_current_stream_capturing():
+        # A list built here would be copied from host memory at every replay,
+        # long after that memory was given back: the padded grid takes the call.
+        return None
     host_k = metadata["host_k_lens"]
     host_off = metadata["host_q_pos_offsets"]
     host_qs = metadata["host_q_starts"]

@@ -1,4 +1,5 @@
-"""What one call keeps for later ones, the step's launch list, on other streams."""
+"""What one call keeps for later ones -- the step's launch list, the stream's
+workspace -- under other streams and under graph capture."""
 import math
 
 import pytest
@@ -66,3 +67,35 @@ def test_a_list_on_other_streams(cuda, sea, wl, hq, hkv, d, dtype):  # noqa: F81
         torch.cuda.synchronize()
         assert_attention(w, o, l, *ref)
         assert (taken[-1] is not None) == ordered
+
+
+@pytest.mark.parametrize("hq,hkv,d,dtype", SHAPES)
+@pytest.mark.parametrize("listed", [False, True])
+def test_captured_calls(cuda, sea, wl, hq, hkv, d, dtype, listed):  # noqa: F811
+    """A step's first call inside a capture, and one after its list was built:
+    every replay, with eager work in between, gives the eager result."""
+    w, ref, meta, call = prepare(sea, wl, hq, hkv, d, dtype, cuda)
+    if listed:
+        call()
+        torch.cuda.synchronize()
+    graphs = []
+    for _ in range(2):
+        announce(f"captured call Hq={hq} Hkv={hkv} D={d} {dtype}, list there {listed}")
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g):
+            out = call()
+        graphs.append((g, out))
+    assert bool(meta.get("_schedules")) == listed
+    for rep in range(3):
+        for g, (o, l) in graphs:
+            o.fill_(float("nan"))
+            l.zero_()
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            announce(f"  replay {rep}")
+            assert_attention(w, o, l, *ref)
+        junk = [torch.full((1 << 20,), 1e30, device=cuda) for _ in range(4)]
+        if rep:
+            assert_attention(w, *call(), *ref)
+        del junk
