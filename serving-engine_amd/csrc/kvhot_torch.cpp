@@ -23,6 +23,7 @@
 #include <ATen/ops/empty.h>
 #include <ATen/ops/empty_like.h>
 #include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include "../../include/kvhot.h"
@@ -188,6 +189,11 @@ struct Attention {
       if (need < 0) return false;
     }
     if (need > 0) {  // the stream's workspace, made by the first call that needs it
+      hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &capture) != hipSuccess)
+        (void)hipGetLastError();
+      if (capture != hipStreamCaptureStatusNone)
+        return false;  // a graph's calls have workspaces of their own
       PyObject* key = Py_BuildValue("(iL)", static_cast<int>(d.index()),
                                     static_cast<long long>(reinterpret_cast<intptr_t>(stream)));
       if (!key) return false;

@@ -46,12 +46,16 @@ DEFAULT_PARTITION_TOKENS = 0
 LIST_UNITS = 8192
 
 # Workspaces are per (device, stream): calls sharing one must be stream-ordered.
+# (Captured calls have one each, in their graph's memory.)
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
 
 
 def _workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor | None:
     if nbytes <= 0:
         return None
+    if torch.cuda.is_current_stream_capturing():
+        # A graph's own: graphs recorded on one stream may be replayed on several.
+        return torch.empty(int(nbytes), dtype=torch.uint8, device=device)
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
     ws = _WORKSPACES.get(key)
     if ws is None or ws.numel() < nbytes:

@@ -73,11 +73,14 @@ def test_a_list_on_other_streams(cuda, sea, wl, hq, hkv, d, dtype):  # noqa: F81
 @pytest.mark.parametrize("listed", [False, True])
 def test_captured_calls(cuda, sea, wl, hq, hkv, d, dtype, listed):  # noqa: F811
     """A step's first call inside a capture, and one after its list was built:
-    every replay, with eager work in between, gives the eager result."""
+    every replay, with eager work in between, gives the eager result, and the
+    graph's workspace is its own."""
+    pak = sea_module("paged_attention_kernel")
     w, ref, meta, call = prepare(sea, wl, hq, hkv, d, dtype, cuda)
     if listed:
         call()
         torch.cuda.synchronize()
+    kept = dict(pak._WORKSPACES)
     graphs = []
     for _ in range(2):
         announce(f"captured call Hq={hq} Hkv={hkv} D={d} {dtype}, list there {listed}")
@@ -85,6 +88,7 @@ def test_captured_calls(cuda, sea, wl, hq, hkv, d, dtype, listed):  # noqa: F811
         with torch.cuda.graph(g):
             out = call()
         graphs.append((g, out))
+    assert {k: v.data_ptr() for k, v in pak._WORKSPACES.items()} == {k: v.data_ptr() for k, v in kept.items()}
     assert bool(meta.get("_schedules")) == listed
     for rep in range(3):
         for g, (o, l) in graphs:
